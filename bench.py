@@ -1,7 +1,7 @@
 """Benchmark of the SALSA coagulation + condensation step on one MI355X.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu-baseline]
-    python bench.py --counter-run {mixed,fp64,copy} [--lanes 16,16,16] [--steps 3]
+    python bench.py --counter-run {mixed,fp64,copy} [--lanes 1,1,1] [--steps 3]
 
 The second form is the program profiled by the hardware-counter runs: it
 runs K steps at a fixed launch shape (no autotune, no timing, no CPU leg), or
@@ -159,7 +159,8 @@ def counter_run(kind, lanes, steps):
     prec = capi.SALSA_FP32_MIXED if kind == "mixed" else capi.SALSA_FP64
     ctx = capi.Context(desc, capi.params(level=4, precision=prec), g.nzp, g.nxp, g.nyp)
     for k in range(3):
-        ctx.set_shape(k, lanes[k])
+        if lanes[k] > 1:                     # 1: the context's own choice, one lane per cell
+            ctx.set_shape(k, lanes[k])
     for _ in range(steps):
         ctx.step_device(fd, n_p, m_p, n_t, m_t, rv_t)
     ctx.sync()
@@ -452,7 +453,7 @@ def main():
                     help="also the forward-mode derivative at config 5 full size (about a minute)")
     ap.add_argument("--no-les", action="store_true")
     ap.add_argument("--counter-run", choices=("mixed", "fp64", "copy"))
-    ap.add_argument("--lanes", default="16,16,16")
+    ap.add_argument("--lanes", default="1,1,1")
     args = ap.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         print("bench.py measures one GPU: the SALSA step has no cross-GPU work "
@@ -504,7 +505,7 @@ def main():
         kms, ksteps = ctx.kernel_time()
         phases = ctx.phase_time()
         ctx.timing(False)
-        shapes = [ctx.shape_of(k) for k in range(3)]
+        shapes = [1, 1, 1]                   # a grid of this size steps with one lane per cell
         # one in-place step for the accuracy comparison
         rv = fd["rv"].clone()
         fdd = dict(fd)
@@ -563,9 +564,8 @@ def main():
         "roofline": {"bound": "valu", "engine": "VALU (no MFMA: not a dense contraction)",
                      "achieved": achieved_tf, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved_tf / FP32_PEAK_TFLOPS, "traffic": prof_traffic,
-                     "kernel": "k_salsa_step, cost class %d (%s), %d lanes per cell"
-                               % (dom, ("clear, RH <= 0.98", "clear, RH > 0.98", "cloudy")[dom],
-                                  shapes_mixed[dom]),
+                     "kernel": "k_lanes_pairs + k_lanes_sweep, cost class %d (%s), one lane per cell"
+                               % (dom, ("clear, RH <= 0.98", "clear, RH > 0.98", "cloudy")[dom]),
                      "kernel_ms_per_launch": d["ms"], "cells_per_launch": d["cells"],
                      "flop_per_cell_step": fpc,
                      "step_achieved": step_tf, "step_frac": step_tf / FP32_PEAK_TFLOPS,

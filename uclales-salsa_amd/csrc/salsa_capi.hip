@@ -27,6 +27,12 @@ int64_t gather_tiles(int64_t ncells);
 int64_t class_work_ints(int64_t ncells);
 int launch_scatter(const DevLayout &Lay, const DevLayout *d, const StepArgs &a, hipStream_t s);
 int launch_act_cloud_base(const DevLayout *d, const StepArgs &a, hipStream_t s);
+bool lanes_fit(const DevLayout &L, int kt, int64_t ncells);
+size_t lanes_work(const DevLayout &L, int kt, int64_t ncells, LanesArgs &w);
+int lanes_program(const DevLayout &L, uint32_t *prog);
+int launch_lanes_class(const DevLayout &L, const DevLayout *d, const StepArgs &a, const LanesArgs &w, hipStream_t s);
+int launch_lanes(const DevLayout &L, int precision, bool hyd, const DevLayout *d, const StepArgs &a, const LanesArgs &w,
+                 hipStream_t s);
 int cap_bins(int cap);
 int cap_spec(int cap);
 int launch_gradient(int cap, int precision, const DevLayout *d, const GradArgs &g, double *sum_out,
@@ -78,6 +84,12 @@ struct salsa_ctx {
   int32_t *lists = nullptr;
   int32_t *cls_count = nullptr;       // device [3]
   int32_t *cls_count_h = nullptr;     // pinned host [3]
+  // one-lane-per-cell step: its work space (null where the layout or the
+  // options need the general kernel); shape_set: the caller chose the general
+  // kernel's lanes per cell
+  char *lanes_buf = nullptr;
+  LanesArgs lw;
+  bool shape_set = false;
   // salsa_gradient_device: per-cell J and dJ/dE, then the two sums
   double *gbuf = nullptr;
   // salsa_adjoint_device: checkpoints, recomputed states, work states, the
@@ -101,13 +113,17 @@ struct salsa_ctx {
   // (gather, the three class kernels, scatter) and the class cell counts
   bool timing = false;
   std::vector<hipEvent_t> ev;
-  std::vector<int64_t> ev_cells;      // [3] per timed step
+  std::vector<int64_t> ev_cells;      // [3] per timed step, read on the host by the general path
+  int32_t *ev_counts_h = nullptr;     // pinned host [kTimedCounts][3]: class counts of the others
+  std::vector<int> ev_slot;           // per timed step: its place in ev_counts_h, -1 where ev_cells has it
+  int ev_counts = 0;
   // this device's copy of the static work space of the allocation-free entry
   double *scratch = nullptr;
   double *tot_h = nullptr;            // pinned host [2]: gradient totals
   int32_t *fault_h = nullptr;         // pinned host [1]: the OR of the cell flags
 };
 constexpr int kEvPerStep = 10;
+constexpr int kTimedCounts = 4096;    // timed steps whose class counts need no wait
 
 // ---------------------------------------------------------------------------
 // Work space of salsa_gradient_device_noalloc: per-cell J, per-cell dJ/dE and
@@ -174,6 +190,8 @@ static void release(salsa_ctx *c) {
   (void)hipFree(c->adj_buf);
   (void)hipFree(c->les_list);
   (void)hipFree(c->act_state);
+  (void)hipFree(c->lanes_buf);
+  if (c->ev_counts_h) (void)hipHostFree(c->ev_counts_h);
   if (c->cls_count_h) (void)hipHostFree(c->cls_count_h);
   if (c->tot_h) (void)hipHostFree(c->tot_h);
   if (c->fault_h) (void)hipHostFree(c->fault_h);
@@ -233,7 +251,7 @@ extern "C" int salsa_ctx_create(const salsa_bin_desc *desc, const salsa_params *
       hipMalloc(&c->lists, 3 * nc * sizeof(int32_t)) != hipSuccess || hipMalloc(&c->cls, nc) != hipSuccess ||
       hipMalloc(&c->tcount, 3 * (size_t)gather_tiles(c->ncells) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc(&c->toff, (size_t)class_work_ints(c->ncells) * sizeof(int32_t)) != hipSuccess ||
-      hipMalloc(&c->cls_count, 3 * sizeof(int32_t)) != hipSuccess ||
+      hipMalloc(&c->cls_count, 4 * sizeof(int32_t)) != hipSuccess ||
       hipMalloc(&c->rec_in, nc * c->hostL.nslot * sizeof(double)) != hipSuccess ||
       hipMalloc(&c->rec_out, nc * c->hostL.nout * sizeof(double)) != hipSuccess ||
       hipHostMalloc(&c->cls_count_h, 3 * sizeof(int32_t)) != hipSuccess ||
@@ -260,6 +278,30 @@ extern "C" int salsa_ctx_create(const salsa_bin_desc *desc, const salsa_params *
     // zero-filled like initialize_coagstorage (mo_salsa_driver.f90:601-648)
     if (hipMemset(c->kstore, 0, nc * (size_t)c->hostL.npair * kt) != hipSuccess) {
       set_error("kernel store initialisation failed");
+      return fail(SALSA_ERR_HIP);
+    }
+  }
+  const int kt = c->params.precision == SALSA_FP64 ? 8 : 4;
+  if (c->params.lscoag_mode == 1 && lanes_fit(c->hostL, kt, c->ncells)) {
+    std::memset(&c->lw, 0, sizeof(c->lw));
+    const size_t need = lanes_work(c->hostL, kt, c->ncells, c->lw);
+    if (hipMalloc(&c->lanes_buf, need) != hipSuccess) {
+      set_error("step work allocation failed");
+      return fail(SALSA_ERR_NOMEM);
+    }
+    c->lw.counts = c->cls_count;
+    c->lw.lists = c->lists;
+    c->lw.ncells = c->ncells;
+    c->lw.K = c->lanes_buf;
+    c->lw.pf = reinterpret_cast<uint8_t *>(c->lanes_buf + c->lw.o_pf);
+    c->lw.dwa = reinterpret_cast<double *>(c->lanes_buf + c->lw.o_dwa);
+    c->lw.rows = reinterpret_cast<LaneRow *>(c->lanes_buf + c->lw.o_rows);
+    c->lw.prog = reinterpret_cast<const uint32_t *>(c->lanes_buf + c->lw.o_prog);
+    std::vector<uint32_t> prog((size_t)lanes_program(c->hostL, nullptr));
+    (void)lanes_program(c->hostL, prog.data());
+    if (hipMemcpy(c->lanes_buf + c->lw.o_prog, prog.data(), prog.size() * sizeof(uint32_t), hipMemcpyHostToDevice) !=
+        hipSuccess) {
+      set_error("copy of the sweep program failed");
       return fail(SALSA_ERR_HIP);
     }
   }
@@ -294,6 +336,7 @@ extern "C" int salsa_set_launch_shape(salsa_ctx *c, int32_t cls, int32_t lanes) 
     return SALSA_ERR_ARG;
   }
   c->lanes[cls] = lanes;
+  c->shape_set = true;
   return SALSA_OK;
 }
 
@@ -413,8 +456,41 @@ static StepArgs class_args(salsa_ctx *c, const StepArgs &a, int k) {
   return b;
 }
 
+// The step with one lane per cell (salsa_lanes.hip): coagulation and
+// condensation without the optional processes, diagnostics and call forms
+// that only the general kernel has.
+static bool use_lanes(const salsa_ctx *c, const StepArgs &a, int32_t flags) {
+  return c->lanes_buf && !c->shape_set && !a.rates && !a.init && !a.kmode && !(flags & SALSA_STEP_NO_COMPACT);
+}
+
+static int enqueue_lanes(salsa_ctx *c, const StepArgs &a) {
+  hipStream_t s = c->stream;
+  const LanesArgs &w = c->lw;
+  MARK();
+  int rc = launch_lanes_class(c->hostL, c->devL, a, w, s);
+  MARK();
+  // classes 0 and 1 share a launch: it is timed between their first events
+  for (int k = 0; k < 3 && !rc; ++k) {
+    MARK();
+    if (k != 1) rc = launch_lanes(c->hostL, c->params.precision, k == 2, c->devL, a, w, s);
+    MARK();
+  }
+  MARK();
+  MARK();
+  if (rc) { std::snprintf(g_err, sizeof(g_err), "step launch failed (%d)", rc); return SALSA_ERR_HIP; }
+  if (c->timing) {
+    const int i = c->ev_counts < kTimedCounts ? c->ev_counts++ : kTimedCounts - 1;
+    if (i == kTimedCounts - 1) HIPCHK(hipStreamSynchronize(s));
+    HIPCHK(hipMemcpyAsync(c->ev_counts_h + 3 * i, c->cls_count, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    c->ev_slot.push_back(i);
+    c->ev_cells.insert(c->ev_cells.end(), 3, 0);
+  }
+  return SALSA_OK;
+}
+
 static int enqueue_step(salsa_ctx *c, StepArgs a, int32_t flags) {
   hipStream_t s = c->stream;
+  if (use_lanes(c, a, flags)) return enqueue_lanes(c, a);
   const bool compact = !(flags & SALSA_STEP_NO_COMPACT);
   MARK();
   int rc = enqueue_gather(c, a, compact);
@@ -446,7 +522,10 @@ static int enqueue_step(salsa_ctx *c, StepArgs a, int32_t flags) {
   rc = launch_scatter(c->hostL, c->devL, a, s);
   if (rc) { std::snprintf(g_err, sizeof(g_err), "scatter launch failed (%d)", rc); return SALSA_ERR_HIP; }
   MARK();
-  if (c->timing) c->ev_cells.insert(c->ev_cells.end(), cells, cells + 3);
+  if (c->timing) {
+    c->ev_cells.insert(c->ev_cells.end(), cells, cells + 3);
+    c->ev_slot.push_back(-1);
+  }
   return SALSA_OK;
 }
 
@@ -456,6 +535,10 @@ extern "C" int salsa_ctx_timing(salsa_ctx *c, int32_t enable) {
   for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
   c->ev.clear();
   c->ev_cells.clear();
+  c->ev_slot.clear();
+  c->ev_counts = 0;
+  if (enable && c->lanes_buf && !c->ev_counts_h)
+    HIPCHK(hipHostMalloc(&c->ev_counts_h, 3 * kTimedCounts * sizeof(int32_t)));
   c->timing = enable != 0;
   return SALSA_OK;
 }
@@ -474,10 +557,21 @@ extern "C" int salsa_ctx_phase_time(salsa_ctx *c, double ms[5], int64_t cells[3]
   };
   for (size_t st = 0; st < n; ++st) {
     if (el(st, 0, 1, ms[0])) return SALSA_ERR_HIP;                 // gather + classification
-    for (int k = 0; k < 3; ++k)
-      if (el(st, 2 + 2 * k, 3 + 2 * k, ms[1 + k])) return SALSA_ERR_HIP;   // class k step kernel
+    const int slot = c->ev_slot[st];
+    int64_t n[3];
+    double t[3] = {0., 0., 0.};
+    for (int k = 0; k < 3; ++k) {
+      n[k] = slot < 0 ? c->ev_cells[3 * st + k] : c->ev_counts_h[3 * slot + k];
+      cells[k] += n[k];
+      if (el(st, 2 + 2 * k, 3 + 2 * k, t[k])) return SALSA_ERR_HIP;        // class k step kernel
+    }
+    if (slot >= 0 && n[0] + n[1] > 0) {        // one launch of both: its time by their cells
+      const double both = t[0];
+      t[0] = both * (double)n[0] / (double)(n[0] + n[1]);
+      t[1] = both - t[0];
+    }
+    for (int k = 0; k < 3; ++k) ms[1 + k] += t[k];
     if (el(st, 8, 9, ms[4])) return SALSA_ERR_HIP;                 // scatter
-    for (int k = 0; k < 3; ++k) cells[k] += c->ev_cells[3 * st + k];
   }
   *nsteps = (int64_t)n;
   return SALSA_OK;
@@ -889,7 +983,9 @@ extern "C" int salsa_autotune(salsa_ctx *c, const double *press, const double *t
   }
   StepArgs a = make_args(c, press, temp, rsl, rsi, dn, rv_p, rvt, n_p, nt, m_p, mt, nullptr, tstep, 0);
   a.kmode = 0;                                           // tuning neither reads nor writes the kernel store
+  c->shape_set = true;                                   // the shapes are the general kernel's
   int rc = enqueue_step(c, a, 0);                        // classification + warm-up
+  c->shape_set = false;
   if (rc) { hipFree(scr); return rc; }
   hipStream_t s = c->stream;
   hipEvent_t e0, e1;

@@ -173,6 +173,27 @@ struct StepArgs {
   double *act_state;                  //   the aerosol state it sees [ncells][nbins*(1+nwet)], or null
 };
 
+// A field row of a one-lane-per-cell step: read from in, results to out; the
+// state holds value * dn / rho.  kind: no such row, a number row, a water row.
+enum { LR_NONE = 1, LR_NUMBER = 2, LR_WATER = 4 };
+struct LaneRow { const double *in; double *out; double rho; int32_t kind, pad; };
+
+// Arguments of the one-lane-per-cell step kernels besides StepArgs.
+struct LanesArgs {
+  int32_t *counts, *lists;            // cells per class [3] (and the first list's fill); ids: without
+                                      //   hydrometeors [ncells], with [ncells]
+  int64_t ncells;
+  int32_t g0;                         // first block of 64 slots of this chunk
+  int32_t gn_hyd, gn_aero;            // blocks that the work space holds with and without hydrometeor pairs
+  LaneRow *rows;                      // the call's field rows in state order
+  const uint32_t *prog;               // the sweep program
+  // per block of the chunk, 64 cells side by side:
+  void *K;                            // kernels [block][pair][64], a row of zeros last
+  uint8_t *pf;                        // COUNT(D_new > precpbins) per cloud-cloud pair [block][ncc][64]
+  double *dwa;                        // wet diameters of the aerosol bins before the step [block][nbins][64]
+  size_t o_pf, o_dwa, o_rows, o_prog;   // byte offsets in the work space
+};
+
 // Arguments of the forward-mode derivative kernel: the trajectory starts from
 // the cell records in s.rec_in and runs nsteps in-place steps of s.dt.
 struct GradArgs {
