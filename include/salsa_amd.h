@@ -340,11 +340,12 @@ int salsa_gradient_device_noalloc(salsa_ctx *ctx, const double *press, const dou
  * (0 = clear and dry, 1 = clear and humid, 2 = cloudy); 0 keeps the current
  * value.  salsa_autotune times the candidates on the given device-resident
  * inputs and keeps the fastest per class.  Large contexts (15 360 cells at
- * level 4, 5 120 at level 5) step with one lane per cell where the layout and
+ * level 4, 4 096 at level 5) step with one lane per cell where the layout and
  * the call allow it (coagulation and condensation only, no rate fields, kernel
- * store or initialization); the shapes then count for the other calls, and
- * salsa_set_launch_shape with a new value selects the shaped kernels for every
- * call of the context. */
+ * store or initialization), and smaller ones in one launch of 16 to 64 lanes
+ * per cell; the shapes then count for the other calls, and
+ * salsa_set_launch_shape with a new value selects launches by cost class with
+ * the shapes for every call of the context. */
 /*
  * The LES side of a SALSA step for the SALSA tracers, on device: what cfll
  * runs after run_SALSA (step.f90:330-333) -- tend_constrain2

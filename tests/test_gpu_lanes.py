@@ -71,7 +71,8 @@ CASES = [
     (("SO4",), 4, (41, 15, 25), 0),
     (("SO4",), 4, (41, 15, 25), 65),
     (("SO4", "DU"), 4, (41, 15, 25), 64),
-    (("SO4",), 5, (40, 8, 16), 63),                  # 5 120 cells: the smallest
+    (("SO4",), 5, (40, 8, 16), 63),
+    (("SO4", "DU"), 5, (32, 8, 16), 63),             # 4 096 cells: the smallest
     (("SO4",), 5, (43, 11, 11), None),
     (("SO4", "DU"), 5, (43, 11, 11), None),
     (("SO4", "DU"), 5, (43, 11, 11), 1),
@@ -117,3 +118,22 @@ def test_one_lane_per_cell_matches_general_kernel(capi, species, level, grid, nh
         rms = np.sqrt(np.mean(y * y, axis=1, keepdims=True))
         bad = ~(np.abs(x - y) <= RTOL * np.abs(y) + ATOL_RMS * rms + 10. * np.abs(y - y2))
         assert not bad.any(), (np.argwhere(bad)[:3], x[bad][:3], y[bad][:3], y2[bad][:3])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("level,grid", [(4, (1, 1, 1)), (4, (13, 5, 1)), (4, (39, 19, 20)), (5, (1, 1, 1)), (5, (33, 3, 7)),
+                                        (5, (31, 11, 11))])
+def test_small_grids_match_the_launches_by_class(capi, level, grid, prec):
+    """Below the sizes of the one-lane path every cell runs in one launch, 32
+    (level 5: 64, above 2 048 cells 16) lanes each: bit for bit what the launches by cost class give
+    at those lanes."""
+    print("case level %d grid %s prec %d" % (level, grid, prec), flush=True)
+    desc, f = fields(capi, ("SO4", "DU"), level, grid)
+    ncat = 4 if level == 5 else 3
+    lanes = 32 if level == 4 else 64 if f.grid.ncells <= 2048 else 16
+    for inplace in (0, 1):
+        a, fa, ea = step(capi, desc, f, prec, f.n[:ncat], f.m[:ncat], f.rv, 0, inplace)
+        b, fb, eb = step(capi, desc, f, prec, f.n[:ncat], f.m[:ncat], f.rv, lanes, inplace)
+        assert ea == eb and np.array_equal(fa, fb)
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)

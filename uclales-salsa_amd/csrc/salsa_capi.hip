@@ -27,6 +27,7 @@ int64_t gather_tiles(int64_t ncells);
 int64_t class_work_ints(int64_t ncells);
 int launch_scatter(const DevLayout &Lay, const DevLayout *d, const StepArgs &a, hipStream_t s);
 int launch_act_cloud_base(const DevLayout *d, const StepArgs &a, hipStream_t s);
+int64_t lanes_least(const DevLayout &L);
 bool lanes_fit(const DevLayout &L, int kt, int64_t ncells);
 size_t lanes_work(const DevLayout &L, int kt, int64_t ncells, LanesArgs &w);
 int lanes_program(const DevLayout &L, uint32_t *prog);
@@ -423,14 +424,33 @@ static int timing_mark(salsa_ctx *c) {
 }
 #define MARK() do { if (timing_mark(c)) return SALSA_ERR_HIP; } while (0)
 
-static int launch_class(salsa_ctx *c, int k, const StepArgs &a, hipStream_t s) {
+static int launch_class(salsa_ctx *c, int k, const StepArgs &a, hipStream_t s, int lanes = 0) {
   const bool hyd = k == 2;
+  if (!lanes) lanes = c->lanes[k];
   SmemGeom G;
-  if (make_geom(c->hostL, hyd, c->params.precision == SALSA_FP64 ? 8 : 4, c->lanes[k], a.rates != nullptr, G)) {
+  if (make_geom(c->hostL, hyd, c->params.precision == SALSA_FP64 ? 8 : 4, lanes, a.rates != nullptr, G)) {
     set_error("launch shape exceeds 64 KiB of LDS per block");
     return SALSA_ERR_ARG;
   }
-  return launch_step(c->cap, c->lanes[k], c->params.precision, hyd, c->devL, a, G, s);
+  return launch_step(c->cap, lanes, c->params.precision, hyd, c->devL, a, G, s);
+}
+
+// Lanes per cell with which a small context runs all its cells in one launch
+// of the variant for hydrometeors; 0 where it goes by cost class.  Classes
+// save work on dry cells, but cost three small kernels, a wait for the counts
+// and launches that follow each other, each as long as its slowest cell: below
+// the size from which one lane per cell pays, the chip has room for every cell
+// at once.  Measured us by class / in one launch: level 4 (32 lanes) mixed
+// 640 cells 198 / 108, 2 560 204 / 119, 10 240 231 / 202, FP64 204 / 113,
+// 208 / 126, 246 / 220; level 5 mixed 640 172 / 152 (64 lanes), 2 560
+// 214 / 193 (64) and 196 (16), 3 840 214 / 256 (64) and 200 (16), FP64 175 /
+// 155, 225 / 204 and 208, 234 / 269 and 212.
+// The kernel store (kmode) keeps its cells in list order and stays by class.
+static int direct_lanes(const salsa_ctx *c, const StepArgs &a) {
+  if (c->shape_set || a.kmode || c->ncells >= lanes_least(c->hostL)) return 0;
+  const int lanes = c->hostL.level == 5 ? (c->ncells <= 2048 ? 64 : 16) : 32;
+  SmemGeom G;
+  return make_geom(c->hostL, true, c->params.precision == SALSA_FP64 ? 8 : 4, lanes, a.rates != nullptr, G) ? 0 : lanes;
 }
 
 // Gather + classification, then the class counts to the host (they size the
@@ -491,7 +511,8 @@ static int enqueue_lanes(salsa_ctx *c, const StepArgs &a) {
 static int enqueue_step(salsa_ctx *c, StepArgs a, int32_t flags) {
   hipStream_t s = c->stream;
   if (use_lanes(c, a, flags)) return enqueue_lanes(c, a);
-  const bool compact = !(flags & SALSA_STEP_NO_COMPACT);
+  const int direct = flags & SALSA_STEP_NO_COMPACT ? 0 : direct_lanes(c, a);
+  const bool compact = !(flags & SALSA_STEP_NO_COMPACT) && !direct;
   MARK();
   int rc = enqueue_gather(c, a, compact);
   if (rc) return rc;
@@ -506,7 +527,7 @@ static int enqueue_step(salsa_ctx *c, StepArgs a, int32_t flags) {
       b = class_args(c, a, k);
     }
     if (b.ncells > 0) {
-      rc = launch_class(c, k, b, s);
+      rc = launch_class(c, k, b, s, direct);
       if (rc) { std::snprintf(g_err, sizeof(g_err), "kernel launch failed (%d)", rc); return SALSA_ERR_HIP; }
     }
     cells[k] = b.ncells;

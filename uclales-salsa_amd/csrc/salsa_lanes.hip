@@ -1129,20 +1129,20 @@ int sweep_program(const DevLayout &L, bool hyd, uint32_t *prog) {
 // 26-bin layout at either size.
 constexpr int kSlotsHyd = 1 << 17, kSlotsAero = 1 << 19;
 
-// Whether the lane kernels take a context of ncells cells with this layout.
-//
-// Below kLeast4 cells (kLeast5 with ice) the general kernel is faster: a
-// workgroup here takes as long for its 64 cells as for one, about 0.1 ms for
-// a sweep, and the chip is filled from 256 workgroups on, while 8 to 64 lanes
-// per cell also share the work of a few cells.  Measured us, here / general:
-// level 4 mixed 5 120 cells 239 / 210, 10 240 243 / 235, 15 360 246 / 269,
-// with drizzle 15 360 264 / 266, 20 480 275 / 288, FP64 10 240 252 / 249,
-// 15 360 256 / 286; level 5 mixed 2 560 233 / 215, 5 120 242 / 247, FP64
-// 2 560 248 / 227, 5 120 255 / 334.
-constexpr int64_t kLeast4 = 15360, kLeast5 = 5120;
+// The fewest cells of a context that steps with one lane per cell.  A
+// workgroup here takes as long for its 64 cells as for one, about 0.1 ms for a
+// sweep, and the chip is filled from 256 workgroups on; 16 to 64 lanes per
+// cell share the work of a few cells.  Measured us, here / the general kernel
+// on all cells in one launch: level 4 (32 lanes) mixed 5 120 cells 239 / 134,
+// 10 240 243 / 202, 15 360 246 / 266, with drizzle 10 240 261 / 215, 15 360
+// 264 / 275, FP64 10 240 252 / 220, 15 360 255 / 292.  Level 5 (16 lanes)
+// mixed 3 840 cells 239 / 200, 5 120 242 / 224, 10 240 254 / 396, FP64 3 840
+// 254 / 212, 5 120 253 / 376: more than one wavefront per SIMD.
+int64_t lanes_least(const DevLayout &L) { return L.level == 5 ? 4096 : 15360; }
 
+// Whether the lane kernels take a context of ncells cells with this layout.
 bool lanes_fit(const DevLayout &L, int kt, int64_t ncells) {
-  if (ncells < (L.level == 5 ? kLeast5 : kLeast4)) return false;
+  if (ncells < lanes_least(L)) return false;
   const int NV = lanes_volumes(L);
   if (NV < 2 || NV > 4 || (NV == 4 && L.level != 5) || (NV == 2 && L.level == 5) || L.nt > 63 || L.npair < 1 || L.npair > 65535) return false;
   const int VL = NV == 2 ? kPart2 : kPart4, bins = VL * (NV == 2 ? kBins2 : kBins4);
