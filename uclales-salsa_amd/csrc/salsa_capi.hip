@@ -1087,6 +1087,7 @@ extern "C" int salsa_les_update_device(salsa_ctx *c, double dtlt, const double *
   a.icb_cur = d.icb.cur; a.icb_par = d.icb.par; a.fcb_cur = d.fcb.cur;
   for (int s = 0; s < SALSA_MAXSPEC; ++s) {
     a.rholiq[s] = d.rholiq[s]; a.rhoice[s] = d.rhoice[s]; a.mm[s] = d.mm[s]; a.diss[s] = d.diss[s];
+    a.rrholiq[s] = 1. / d.rholiq[s]; a.diss_mm[s] = d.diss[s] / d.mm[s];
   }
   for (int b = 0; b < d.nbins; ++b) a.aerobins[b] = std::pow(d.vlolim[b] / 0.5235988, 1. / 3.);   // set_aerobins
   a.temp = temp; a.rh = rh; a.rhi = rhi ? rhi : rh; a.rp = rp;

@@ -256,6 +256,7 @@ struct LesArgs {
   int32_t in1a, fn2b, in2a, fn2a;
   int32_t ica_cur, ica_par, fca_cur, icb_cur, icb_par, fcb_cur;
   double rholiq[kMaxSpec], rhoice[kMaxSpec], mm[kMaxSpec], diss[kMaxSpec];
+  double rrholiq[kMaxSpec], diss_mm[kMaxSpec];   // 1 / rholiq, diss / mm
   double aerobins[kMaxBin];           // lower dry-diameter limit of each aerosol bin
   const double *temp, *rh, *rhi, *rp;
   double *n_p[4], *n_t[4], *m_p[4], *m_t[4];

@@ -2,28 +2,23 @@
 // after run_SALSA (step.f90:330-333) for the SALSA tracers, so that the
 // prognostic fields never leave HBM between steps.
 //
-//   pass A  tend_constrain2 (constrain_SALSA.f90:18-36; a_indefp clamped
-//           when registered), update
-//           (step.f90:470-489) on the interior, tend0 (step.f90:379-396):
-//           one thread per array element, rows streamed contiguously, one
-//           launch over the rows of every category.
-//   pass B  sclrset 'mixd' (util.f90:71-107): the bottom row copies k = 2,
-//           the top row extrapolates with dzf2 = dzt(nzp-2)/dzt(nzp-1); the
-//           lateral halos are the periodic images (cyclics/cyclicc of a
-//           process that owns the whole grid).  One launch over every row:
-//           one thread per (halo column, level) or per interior column.
-//   pass D  SALSA_diagnostics (constrain_SALSA.f90:50-402): clamps on every
-//           cell; on interior columns the removal of particles with number
-//           but no mass, cloud / precipitation / ice bins that evaporated
-//           back to the aerosol bins (findDry4Wet :408-470 for
-//           precipitation and ice), aerosols below 0.1 nm dry diameter; then
-//           the diagnostic sums rc, srp, snrp, rtot, ri, riri on every cell.
-//           One thread per cell; per cell the bins are visited in the
-//           reference's order, so the result does not depend on the grid
-//           traversal.  A streaming part reads each row once (clamps,
-//           sums, and whether any removal test holds, listing those cells);
-//           the removals then run on the listed cells only, with each
-//           cell's rows staged in LDS where they fit.
+//   k_les_cells   interior columns, one lane per cell, every row once:
+//                 tend_constrain2 (constrain_SALSA.f90:18-36), update
+//                 (step.f90:470-489), tend0 (step.f90:379-396), the bottom and
+//                 top rows of sclrset 'mixd' (util.f90:71-107: the bottom
+//                 copies k = 2, the top extrapolates with dzf2 =
+//                 dzt(nzp-2)/dzt(nzp-1)), SALSA_diagnostics' clamps
+//                 (constrain_SALSA.f90:88-100) and diagnostic sums (:370-400),
+//                 and a list of the cells that its removals may change;
+//                 a column at an edge writes its periodic images too
+//                 (cyclics/cyclicc of a process that owns the whole grid).
+//   k_les_remove  SALSA_diagnostics' removals (:103-366) on the listed cells:
+//                 particles with number but no mass, cloud / precipitation /
+//                 ice bins that evaporated back to the aerosol bins
+//                 (findDry4Wet :408-470 for precipitation and ice), aerosols
+//                 below 0.1 nm dry diameter; each cell's rows staged in LDS
+//                 where they fit, the bins in the reference's order.
+//   k_les_start   the list empty; a_indefp clamped when registered (:33-34).
 //
 // The passes are HBM-bound byte movers, coalesced along k (the fastest LES
 // index).  Floating-point contraction is off so that every sum
@@ -43,111 +38,14 @@ namespace salsa {
 namespace {
 
 constexpr double kMassTH = 1.e-25;    // constrain_SALSA.f90:65
-constexpr int kLesGroup = 2;          // bins whose rows the diagnostics pass loads together
 constexpr int kLesCells = 64;         // listed cells per workgroup of the LDS removal pass
 constexpr int kLesLdsRows = 128;      // rows per cell that fit its 64 KiB of LDS
 
-__device__ __forceinline__ bool interior_col(const LesArgs &a, int i, int j) {
-  return i >= 2 && i <= a.nxp - 3 && j >= 2 && j <= a.nyp - 3;
-}
-
-// Row r of the concatenated tracer rows of every category (number rows, then
-// mass rows, category by category): its prognostic and tendency rows.  The
-// same for every thread of a workgroup (r is blockIdx.y).  Rows past the
-// tracers: the a_indefp rows of the update pass (t null).
-__device__ __forceinline__ void les_row(const LesArgs &a, int r, double *&p, double *&t) {
-  const int ncat = a.level == 5 ? 4 : 3;
-  p = t = nullptr;
-  for (int c = 0; c < ncat; ++c) {
-    if (r < a.nb[c]) {
-      p = a.n_p[c] + (int64_t)r * a.n3;
-      t = a.n_t[c] + (int64_t)r * a.n3;
-      return;
-    }
-    r -= a.nb[c];
-    const int nm = a.nb[c] * a.nsw[c];
-    if (r < nm) {
-      p = a.m_p[c] + (int64_t)r * a.n3;
-      t = a.m_t[c] + (int64_t)r * a.n3;
-      return;
-    }
-    r -= nm;
-  }
-  if (a.indef && r < a.nindef) p = a.indef + (int64_t)r * a.n3;
-}
-
-// pass A, every tracer row in one launch: blockIdx.y the row, x the cell
-__global__ void __launch_bounds__(256) k_les_update(LesArgs a) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= (int)a.n3) return;
-  double *p, *t;
-  les_row(a, (int)blockIdx.y, p, t);
-  if (!p) return;
-  const int k = x % a.nzp, col = x / a.nzp;
-  const int i = col % a.nxp, j = col / a.nxp;
-  if (x == 0 && blockIdx.y == 0) *a.count = 0; // the removal list of this call starts empty
-  if (!t) {                                   // tend_constrain2's a_indefp clamp (:33-34)
-    p[x] = fmin(fmax(p[x], 0.), 1.);
-    return;
-  }
-  const double rdt = a.dtlt;
-  const double pv = p[x], tv = t[x];
-  const double tc = fmax((-1. + 1.e-8) * pv / rdt, tv);
-  if (k >= 1 && k <= a.nzp - 2 && interior_col(a, i, j)) p[x] = pv + tc * rdt;
-  t[x] = 0.;
-}
-
-// pass B, every tracer row in one launch, blockIdx.y the row.  Workgroups
-// below gh fill the halo columns: one thread per (halo column, k), k fastest,
-// so a wavefront reads and writes along one column; the halo columns are the
-// 2 rows of columns at each y edge (all x) followed by the 2 columns at each x
-// edge of the interior y range.  The others set the bottom and top rows of
-// the interior columns (sclrset 'mixd'), one thread per column.  The halo
-// reads interior levels 1 .. nzp-2 only, which the bottom / top rows leave
-// alone, so the two parts need no order.
-__global__ void __launch_bounds__(256) k_les_bound(LesArgs a, unsigned gh) {
-  double *p, *t;
-  les_row(a, (int)blockIdx.y, p, t);
-  if (!t) return;
-  const int nz = a.nzp, nxp = a.nxp, nyp = a.nyp, nx = nxp - 4, ny = nyp - 4;
-  if (blockIdx.x < gh) {
-    const int nhc = 4 * nxp + 4 * ny;
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nhc * nz) return;
-    const int hc = h / nz, k = h % nz;
-    int i, j;
-    if (hc < 4 * nxp) {
-      const int jq = hc / nxp;
-      j = jq < 2 ? jq : nyp - 4 + jq;
-      i = hc % nxp;
-    } else {
-      const int q = (hc - 4 * nxp) % 4;
-      j = 2 + (hc - 4 * nxp) / 4;
-      i = q < 2 ? q : nxp - 4 + q;
-    }
-    const int ii = i < 2 ? i + nx : (i > nxp - 3 ? i - nx : i);
-    const int jj = j < 2 ? j + ny : (j > nyp - 3 ? j - ny : j);
-    const double *src = p + ((int64_t)ii + (int64_t)nxp * jj) * nz;
-    double v;
-    if (k == 0) {
-      const double s1 = src[1], s2 = src[2];
-      v = s1 - 0. * (s2 - s1);
-    } else if (k == nz - 1) {
-      const double sm = src[nz - 2], sm2 = src[nz - 3];
-      v = sm + a.dzf2 * (sm - sm2);
-    } else {
-      v = src[k];
-    }
-    p[((int64_t)i + (int64_t)nxp * j) * nz + k] = v;
-  } else {
-    const int c = (blockIdx.x - gh) * blockDim.x + threadIdx.x;
-    if (c >= nx * ny) return;
-    const int i = 2 + c % nx, j = 2 + c / nx;
-    double *col = p + ((int64_t)i + (int64_t)nxp * j) * nz;
-    const double s1 = col[1], s2 = col[2], sm = col[nz - 2], sm2 = col[nz - 3];
-    col[0] = s1 - 0. * (s2 - s1);
-    col[nz - 1] = sm + a.dzf2 * (sm - sm2);
-  }
+// The list of this call starts empty; a_indefp to [0, 1] (tend_constrain2, :33-34).
+__global__ void __launch_bounds__(256) k_les_start(LesArgs a, int64_t nind) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.count = 0;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nind; e += (int64_t)gridDim.x * blockDim.x)
+    a.indef[e] = fmin(fmax(a.indef[e], 0.), 1.);
 }
 
 // One cell's tracer rows, either in the LES arrays (row stride n3) or staged
@@ -365,148 +263,258 @@ __device__ __forceinline__ void les_sums(const LesArgs &a, const LesCell &C, int
   a.diag[3 * n3 + x] = rtot;
 }
 
-__device__ __forceinline__ bool les_interior_cell(const LesArgs &a, int64_t x) {
-  const int64_t col = x / a.nzp;
-  return interior_col(a, (int)(col % a.nxp), (int)(col / a.nxp));
+// Whether a wet bin (number n, masses m) can pass les_remove's evaporation test
+// zdh2o < min(f * critical diameter, d) || water < kMassTH * n: the cubes of the
+// diameters, which need no power, with a margin far above their rounding.
+template <int MS>
+__device__ __forceinline__ bool les_may_dry(const LesArgs &a, double n, const double (&m)[MS], double T, double f3,
+                                            double d3) {
+  double ns = 0., zvol = 0., wv = 0.;
+#pragma unroll
+  for (int s = 0; s < MS; ++s) {
+    if (s < a.ndry) ns = ns + a.diss_mm[s] * m[s];
+    if (s < a.nwet) zvol = zvol + m[s] * a.rrholiq[s];
+    if (s == a.iwa) wv = m[s];
+  }
+  const double c2 = (4.5 * kRg / (kPi * kSurfw0)) * T * (ns / n);      // critical diameter squared
+  return zvol < fmin(f3 * (c2 * ::sqrt(c2)), d3) * (kPi6 * (1. + 1.e-9)) * n || wv < kMassTH * n;
 }
 
-// pass D, streaming part: one thread per cell, the bins of each category in
-// groups of kLesGroup whose rows (number and every mass species) are loaded
-// together.  Clamps (written where they change a value), the diagnostic
-// sums in bin order, and for interior cells whether any removal test of
-// les_remove holds on the clamped values: its outer conditions, which are
-// what it tests first on values nothing has changed yet (false means
-// les_remove would leave the cell as it is).  Each row is read once.  MS:
-// the most mass rows per bin of any category (registers per bin).
+// Wavefronts of a column, each with an even share of its levels (of 4 and
+// more: no share splits the three lowest or the three highest levels).
+__host__ __device__ inline int les_chunks(int nzp) { return (nzp + 127) / 128; }
+
+constexpr int kLesWaves = 4;                  // wavefronts per workgroup
+
+// two neighbouring levels of a row, on any 8-byte boundary
+typedef double les2 __attribute__((ext_vector_type(2)));
+typedef les2 les2u __attribute__((aligned(8)));
+
+// Interior columns: two neighbouring levels per lane, a wavefront per chunk of
+// a column, bin after bin, the next bin's rows (number, every mass species,
+// their tendencies) loaded before the current one's are stored.  Per row: the
+// tendency floored and added, the bottom and top levels from their two
+// neighbours (read lane to lane, before the clamps), the clamp, the new value
+// and a zero tendency stored, at an edge also to the periodic images; per bin
+// the diagnostic sums in bin order and whether any removal test of les_remove
+// can hold on the clamped values (its conditions as it meets them on values
+// nothing has changed yet, with a margin where they are formed otherwise: false
+// means that it would leave the cell as it is).  MS: the mass rows of an ice
+// bin, one more than a liquid bin has.
+//
+// HBM-bound: 32 B per element, each row touched once (1.42 GB at 64 x 64 x 120
+// cells, 338 us, 4.2 TB/s; as passes for the update, the bottom and top rows
+// and halos, the sums and the removals 212 + 48 + 132 + 65 us).  The loop body has no
+// branch around a load or store (lanes past the chunk, and the last of an odd
+// one, repeat its last two levels; edge columns take another copy of the loop):
+// a wait then leaves the stores behind it in flight, which a count that differs
+// by path would not.  Two levels per lane halve the changes of row, each of
+// which is another page.
 template <int MS>
-__global__ void __launch_bounds__(256) k_les_diag(LesArgs a) {
+__global__ void __launch_bounds__(64 * kLesWaves) k_les_cells(LesArgs a) {
   const int ncat = a.level == 5 ? 4 : 3;
-  const int iwa = a.iwa, irim = a.irim, nwet = a.nwet, ndry = a.ndry;
+  constexpr int iwa = MS - 2, irim = MS - 1, nwet = MS - 1, ndry = MS - 2;
   const int64_t n3 = a.n3;
-  for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < n3; x += (int64_t)gridDim.x * blockDim.x) {
-    const bool inter = les_interior_cell(a, x);
-    const double rh = a.rh[x], rhi = a.level == 5 ? a.rhi[x] : 0.;
-    bool any = false;
-    double sa = 0., sc = 0., sp = 0., sn = 0., si = 0., sr = 0.;
-    // groups of kLesGroup bins, categories in order; the next group's rows
-    // are loaded before the current group's clamps are stored (different
-    // rows), so two groups of loads are in flight
-    double vn[2][kLesGroup], vm[2][kLesGroup][MS];
-    auto load = [&](int c, int b0, double (&n)[kLesGroup], double (&m)[kLesGroup][MS]) {
-      const int nb = a.nb[c], nsw = a.nsw[c];
-      const double *np = a.n_p[c] + x, *mp = a.m_p[c] + x;
+  const int nx = a.nxp - 4, ny = a.nyp - 4, nch = les_chunks(a.nzp);
+  const int lane = threadIdx.x & 63;
+  const int unit = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kLesWaves + threadIdx.x / 64));
+  if (unit >= nx * ny * nch) return;
+  // the rows of columns at the y edges first: they have the most images
+  const int q = unit / nch, h = unit % nch, i = 2 + q % nx, j = 2 + (q / nx + ny - 2) % ny;
+  const int k0 = (int)((int64_t)h * a.nzp / nch), nlev = (int)((int64_t)(h + 1) * a.nzp / nch) - k0;
+  const int kk = 2 * lane < nlev - 2 ? 2 * lane : nlev - 2;      // this lane's two levels from k0
+  const bool in0 = k0 + kk >= 1, in1 = k0 + kk + 1 <= a.nzp - 2; // interior (nzp >= 4: one end each)
+  const bool first = h == 0, last = h == nch - 1;
+  const bool bot = k0 + kk == 0, top = k0 + kk == a.nzp - 2;
+  const int lt = (nlev + 1) / 2 - 1;          // the lane of the last two levels
+  const int64_t x = ((int64_t)i + (int64_t)a.nxp * j) * a.nzp + k0 + kk;
+  // the column's periodic images in the halo: bit 3 v + u for the one shifted by
+  // u - 1 domains along x and v - 1 along y (several on the smallest grids)
+  const int64_t sx = (int64_t)nx * a.nzp, sy = (int64_t)a.nxp * ny * a.nzp;
+  const uint32_t ux = (i - nx >= 0 ? 1u : 0u) | 2u | (i + nx < a.nxp ? 4u : 0u);
+  const uint32_t vy = (j - ny >= 0 ? 1u : 0u) | 2u | (j + ny < a.nyp ? 4u : 0u);
+  const uint32_t im = ((vy & 1u) ? ux : 0u) | (ux & ~2u) << 3 | ((vy & 4u) ? ux << 6 : 0u);
+  auto images = [&](auto &&f) {
+    for (uint32_t left = im; left; left &= left - 1) {
+      const int e = __builtin_ctz(left);
+      f((e % 3 - 1) * sx + (e / 3 - 1) * sy);
+    }
+  };
+  auto get = [](const double *p) -> les2 { return *(const les2u *)p; };
+  auto set = [](double *p, les2 v) { *(les2u *)p = v; };
+  const les2 zero = {0., 0.};
+  const les2 rh = get(a.rh + x), rhi = a.level == 5 ? get(a.rhi + x) : zero, T = get(a.temp + x);
+  const double rdt = a.dtlt;
+  auto from = [](double v, int l) -> double {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
+  };
+  // the new values of a row of which this lane holds p and t (:18-36, step.f90:470-489, util.f90:71-107), clamped
+  auto fresh = [&](les2 pv, les2 tv) -> les2 {
+    // the floor is rarely reached: its division only where it is close
+    const les2 lo = (-1. + 1.e-8) * pv;
+    const bool f0 = tv.x * rdt >= lo.x + fabs(lo.x) * 1.e-12, f1 = tv.y * rdt >= lo.y + fabs(lo.y) * 1.e-12;
+    les2 tc = tv;
+    if (__any(!f0 || !f1)) {
+      tc.x = f0 ? tv.x : fmax(lo.x / rdt, tv.x);
+      tc.y = f1 ? tv.y : fmax(lo.y / rdt, tv.y);
+    }
+    les2 v;
+    v.x = in0 ? pv.x + tc.x * rdt : pv.x;
+    v.y = in1 ? pv.y + tc.y * rdt : pv.y;
+    les2 o = v;
+    if (first) {
+      const double s1 = from(v.y, 0), s2 = from(v.x, 1);
+      if (bot) o.x = s1 - 0. * (s2 - s1);
+    }
+    if (last) {
+      const double sm = from(v.x, lt), sm2 = nlev & 1 ? from(v.x, lt - 1) : from(v.y, lt - 1);
+      if (top) o.y = sm + a.dzf2 * (sm - sm2);
+    }
+    o.x = o.x >= 0. ? o.x : fmax(0., o.x);
+    o.y = o.y >= 0. ? o.y : fmax(0., o.y);
+    return o;
+  };
+  bool any[2] = {false, false};
+  les2 sa = zero, sc = zero, sp = zero, sn = zero, si = zero, sr = zero;
+  struct Bin { les2 n, nt, m[MS], mt[MS]; };
+  // bin b of category c
+  auto load = [&](int c, int b, Bin &B) {
+    const int nb = a.nb[c], nsw = MS - 1 + (c == 3);
+    const int64_t o = (int64_t)b * n3 + x;
+    B.n = get(a.n_p[c] + o);
+    B.nt = get(a.n_t[c] + o);
 #pragma unroll
-      for (int u = 0; u < kLesGroup; ++u) {
-        const int b = b0 + u;
-        n[u] = b < nb ? np[(int64_t)b * n3] : 0.;
+    for (int s = 0; s < MS; ++s) {
+      // (a liquid bin has no rime row: that place repeats its water)
+      const int64_t r = (int64_t)((s < nsw ? s : nsw - 1) * nb) * n3 + o;
+      B.m[s] = get(a.m_p[c] + r);
+      B.mt[s] = get(a.m_t[c] + r);
+    }
+  };
+  auto run = [&](auto edge) {
+    Bin B, F;
+    // category c is a constant, so that every sum stays in its register
+    auto category = [&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+      const int nb = a.nb[c], nsw = MS - 1 + (c == 3);
+      for (int b = 0; b < nb; ++b) {
+        const bool more = b + 1 < nb;
+        int cn = more ? c : c + 1;
+        while (cn < ncat && cn != c && a.nb[cn] == 0) ++cn;
+        load(cn < ncat ? cn : c, cn < ncat ? (more ? b + 1 : 0) : b, F);
+        const les2 n2 = fresh(B.n, B.nt);
+        les2 m2[MS];
 #pragma unroll
-        for (int s = 0; s < MS; ++s) m[u][s] = b < nb && s < nsw ? mp[((int64_t)s * nb + b) * n3] : 0.;
-      }
-    };
-    int c = 0, b0 = 0;
-    load(0, 0, vn[0], vm[0]);
-    // one group; the buffer index is a template constant (no dynamic
-    // register index), the loop below alternates the two
-    auto group = [&](auto cur_c) -> bool {
-      constexpr int cur = decltype(cur_c)::value;
-      int c1 = c, b1 = b0 + kLesGroup;
-      if (b1 >= a.nb[c]) { c1 = c + 1; b1 = 0; }
-      const bool more = c1 < ncat;
-      if (more) load(c1, b1, vn[cur ^ 1], vm[cur ^ 1]);
-      const int nb = a.nb[c], nsw = a.nsw[c];
-      double *np = a.n_p[c] + x, *mp = a.m_p[c] + x;
-      double (&n_)[kLesGroup] = vn[cur];
-      double (&m_)[kLesGroup][MS] = vm[cur];
-      // remove negative values (:88-100); only values that change are written
+        for (int s = 0; s < MS; ++s) m2[s] = s < nsw ? fresh(B.m[s], B.mt[s]) : zero;
+        auto put = [&](int64_t y) {
+          const int64_t o = (int64_t)b * n3 + y;
+          set(a.n_p[c] + o, n2);
+          set(a.n_t[c] + o, zero);
 #pragma unroll
-      for (int u = 0; u < kLesGroup; ++u) {
-        const int b = b0 + u;
-        if (b >= nb) continue;
-        if (!(n_[u] >= 0.)) {
-          n_[u] = fmax(0., n_[u]);
-          np[(int64_t)b * n3] = n_[u];
-        }
-#pragma unroll
-        for (int s = 0; s < MS; ++s)
-          if (s < nsw && !(m_[u][s] >= 0.)) {
-            m_[u][s] = fmax(0., m_[u][s]);
-            mp[((int64_t)s * nb + b) * n3] = m_[u][s];
-          }
-      }
-#pragma unroll
-      for (int u = 0; u < kLesGroup; ++u) {
-        const int b = b0 + u;
-        if (b >= nb) continue;
-        const double n = n_[u];
-        double wv = 0., rv = 0.;                // water and rime masses (no dynamic register index)
+          for (int s = 0; s < MS; ++s)
+            if (s < nsw) {
+              set(a.m_p[c] + ((int64_t)(s * nb) * n3 + o), m2[s]);
+              set(a.m_t[c] + ((int64_t)(s * nb) * n3 + o), zero);
+            }
+        };
+        put(x);
+        if constexpr (decltype(edge)::value) images([&](int64_t o) { put(x + o); });
+        les2 wv = zero, rv = zero;            // water and rime masses (no dynamic register index)
 #pragma unroll
         for (int s = 0; s < MS; ++s) {
-          if (s == iwa) wv = m_[u][s];
-          if (s == irim) rv = m_[u][s];
+          if (s == iwa) wv = m2[s];
+          if (s == irim) rv = m2[s];
         }
-        if (c < 2) {
-          double sm = 0.;
 #pragma unroll
-          for (int s = 0; s < MS; ++s)
-            if (s < nwet) sm = sm + m_[u][s];
-          any |= n > 0. && sm <= 0.;
+        for (int u = 0; u < 2; ++u) {
+          const double n = n2[u];
+          double m[MS];
+#pragma unroll
+          for (int s = 0; s < MS; ++s) m[s] = m2[s][u];
+          if constexpr (c < 2) {
+            double sm = 0.;
+#pragma unroll
+            for (int s = 0; s < MS; ++s)
+              if (s < nwet) sm = sm + m[s];
+            any[u] |= n > 0. && sm <= 0.;
+          }
+          if constexpr (c == 0) {
+            double zvol = 0.;
+#pragma unroll
+            for (int s = 0; s < MS; ++s)
+              if (s < ndry) zvol = zvol + m[s] * a.rrholiq[s];
+            any[u] |= n > kNlim && zvol < (kPi6 * 1.e-30 * (1. + 1.e-9)) * n;
+          } else if constexpr (c == 1) {
+            if (b >= a.ica_cur && b <= a.fcb_cur && rh[u] < 0.999 && n > kNlim && wv[u] < 1.e-5)
+              any[u] |= les_may_dry<MS>(a, n, m, T[u], 0.343, 2.197e-15);
+          } else if constexpr (c == 2) {
+            any[u] |= n > 0. && wv[u] <= 0.;
+            if (rh[u] < 0.999 && n > kPrlim && wv[u] < 1.e-6) any[u] |= les_may_dry<MS>(a, n, m, T[u], 0.008, 1.e-15);
+          } else {
+            const double mt = wv[u] + rv[u];
+            any[u] |= n > 0. && mt < kMassTH;
+            any[u] |= n > kPrlim && rhi[u] < 0.999 && mt < 1.e-15;
+          }
         }
-        if (c == 0) {
-          double zvol = 0.;
-#pragma unroll
-          for (int s = 0; s < MS; ++s)
-            if (s < ndry) zvol = zvol + m_[u][s] / a.rholiq[s];
-          any |= n > kNlim && zvol / n < kPi6 * 1.e-30;
+        if constexpr (c == 0) {
           if (b >= a.in1a && b <= a.fn2b) sa = sa + wv;
-        } else if (c == 1) {
-          any |= b >= a.ica_cur && b <= a.fcb_cur && rh < 0.999 && n > kNlim && wv < 1.e-5;
+        } else if constexpr (c == 1) {
           if (b >= a.ica_cur && b <= a.fcb_cur) sc = sc + wv;
-        } else if (c == 2) {
-          any |= n > 0. && wv <= 0.;
-          any |= rh < 0.999 && n > kPrlim && wv < 1.e-6;
+        } else if constexpr (c == 2) {
           sp = sp + wv;
-          sn = sn + n;
+          sn = sn + n2;
         } else {
-          const double mt = wv + rv;
-          any |= n > 0. && mt < kMassTH;
-          any |= n > kPrlim && rhi < 0.999 && mt < 1.e-15;
           si = si + wv;
           sr = sr + rv;
         }
+        B = F;
       }
-      c = c1;
-      b0 = b1;
-      return more;
     };
-    while (group(std::integral_constant<int, 0>{}) && group(std::integral_constant<int, 1>{})) {
-    }
-    // diagnostic tracers (:370-400), as les_sums forms them
-    const double rc = sa + sc;
-    double rtot = rc + sp + a.rp[x];
-    a.diag[x] = rc;
-    a.diag[n3 + x] = sp;
-    a.diag[2 * n3 + x] = sn;
-    if (a.level == 5) {
-      rtot = rtot + si + sr;
-      a.diag[4 * n3 + x] = si;
-      a.diag[5 * n3 + x] = sr;
-    }
-    a.diag[3 * n3 + x] = rtot;
-    // append the cell to the list of cells the removals visit (one atomic
-    // per wavefront; the list order does not matter, cells are independent)
-    const bool fl = inter && any;
-    const unsigned long long bal = __ballot(fl);
-    if (bal) {
-      const int lane = (int)__lane_id(), leader = __ffsll((long long)bal) - 1;
-      int base = 0;
-      if (lane == leader) base = atomicAdd(a.count, (int)__popcll(bal));
-      base = __shfl(base, leader);
-      if (fl) a.list[base + (int)__popcll(bal & ((1ull << lane) - 1ull))] = (int32_t)x;
-    }
+    int c0 = 0;
+    while (c0 < ncat - 1 && a.nb[c0] == 0) ++c0;
+    load(c0, 0, B);
+    category(std::integral_constant<int, 0>{});
+    category(std::integral_constant<int, 1>{});
+    category(std::integral_constant<int, 2>{});
+    if (ncat == 4) category(std::integral_constant<int, 3>{});
+  };
+  if (im) run(std::true_type{});
+  else run(std::false_type{});
+  // diagnostic tracers (:370-400), as les_sums forms them
+  {
+    const les2 rc = sa + sc;
+    auto sums = [&](int64_t y) {
+      les2 rtot = rc + sp + get(a.rp + y);
+      set(a.diag + y, rc);
+      set(a.diag + n3 + y, sp);
+      set(a.diag + 2 * n3 + y, sn);
+      if (a.level == 5) {
+        rtot = rtot + si + sr;
+        set(a.diag + 4 * n3 + y, si);
+        set(a.diag + 5 * n3 + y, sr);
+      }
+      set(a.diag + 3 * n3 + y, rtot);
+    };
+    sums(x);
+    images([&](int64_t o) { sums(x + o); });
+  }
+  // append the cells to the list of cells the removals visit (one atomic
+  // per wavefront; the list order does not matter, cells are independent)
+  const bool own = 2 * lane < nlev;           // the lanes past it repeat levels, as does the first of a last odd one
+  const bool fl0 = own && kk == 2 * lane && any[0], fl1 = own && any[1];
+  const unsigned long long m0 = __ballot(fl0), m1 = __ballot(fl1);
+  if (m0 | m1) {
+    const int n0 = (int)__popcll(m0);
+    int base = 0;
+    if (lane == 0) base = atomicAdd(a.count, n0 + (int)__popcll(m1));
+    base = __builtin_amdgcn_readfirstlane(base);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (fl0) a.list[base + (int)__popcll(m0 & below)] = (int32_t)x;
+    if (fl1) a.list[base + n0 + (int)__popcll(m1 & below)] = (int32_t)(x + 1);
   }
 }
 
-// pass D, removals on the listed cells, on the LES arrays (layouts whose
+// Removals on the listed cells, on the LES arrays (layouts whose
 // rows do not fit kLesLdsRows); their sums are formed again from the final
 // values
 __global__ void __launch_bounds__(256) k_les_remove(LesArgs a) {
@@ -526,7 +534,7 @@ __global__ void __launch_bounds__(256) k_les_remove(LesArgs a) {
   }
 }
 
-// pass D, removals on the listed cells with each cell's rows staged in LDS
+// Removals on the listed cells with each cell's rows staged in LDS
 // (one lane per listed cell, its own column lds[row * kLesCells + lane]):
 // the sequence of dependent tests runs at LDS latency.  A cell whose
 // removals changed something writes all its rows back and its sums again.
@@ -595,21 +603,17 @@ int launch_les_update(const LesArgs &a, hipStream_t s) {
   const int ncat = a.level == 5 ? 4 : 3;
   int nrow = 0;
   for (int c = 0; c < ncat; ++c) nrow += a.nb[c] * (1 + a.nsw[c]);
-  const int nind = a.indef && a.level == 5 ? a.nindef : 0;
-  if (nrow < 1 || nrow + nind > 65535) return (int)hipErrorInvalidValue;
-  const unsigned gx = (unsigned)((a.n3 + 255) / 256);
-  hipLaunchKernelGGL(k_les_update, dim3(gx, nrow + nind), dim3(256), 0, s, a);
-  const unsigned gh = (unsigned)(((4 * a.nxp + 4 * (a.nyp - 4)) * a.nzp + 255) / 256);
-  const unsigned gr = (unsigned)(((a.nxp - 4) * (a.nyp - 4) + 255) / 256);
-  hipLaunchKernelGGL(k_les_bound, dim3(gh + gr, nrow), dim3(256), 0, s, a, gh);
-  int msw = 0;
-  for (int c = 0; c < ncat; ++c) msw = a.nsw[c] > msw ? a.nsw[c] : msw;
-  if (msw <= 3)
-    hipLaunchKernelGGL(k_les_diag<3>, dim3(grid_for(a.n3, 256)), dim3(256), 0, s, a);
-  else if (msw <= 5)
-    hipLaunchKernelGGL(k_les_diag<5>, dim3(grid_for(a.n3, 256)), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(k_les_diag<kMaxSpec>, dim3(grid_for(a.n3, 256)), dim3(256), 0, s, a);
+  const int64_t nind = a.indef && a.level == 5 ? (int64_t)a.nindef * a.n3 : 0;
+  hipLaunchKernelGGL(k_les_start, dim3(grid_for(nind, 256)), dim3(256), 0, s, a, nind);
+  // what k_les_cells takes for granted of a layout: one or two dry species, water, rime
+  const int ms = a.nsw[0] + 1;
+  if (ms < 3 || ms > 4 || a.nsw[1] != ms - 1 || a.nsw[2] != ms - 1 || (ncat == 4 && a.nsw[3] != ms) ||
+      a.nwet != ms - 1 || a.ndry != ms - 2 || a.iwa != ms - 2 || (ncat == 4 && a.irim != ms - 1))
+    return (int)hipErrorInvalidValue;
+  const int64_t units = (int64_t)(a.nxp - 4) * (a.nyp - 4) * les_chunks(a.nzp);
+  const dim3 gc((unsigned)((units + kLesWaves - 1) / kLesWaves)), tc(64 * kLesWaves);
+  if (ms == 3) hipLaunchKernelGGL(k_les_cells<3>, gc, tc, 0, s, a);
+  else hipLaunchKernelGGL(k_les_cells<4>, gc, tc, 0, s, a);
   if (nrow <= kLesLdsRows) {
     const int64_t g = (a.n3 + kLesCells - 1) / kLesCells;
     hipLaunchKernelGGL(k_les_remove_lds, dim3((unsigned)(g < 4096 ? g : 4096)), dim3(kLesCells),
