@@ -284,41 +284,45 @@ __device__ __forceinline__ bool les_may_dry(const LesArgs &a, double n, const do
 // more: no share splits the three lowest or the three highest levels).
 __host__ __device__ inline int les_chunks(int nzp) { return (nzp + 127) / 128; }
 
-constexpr int kLesWaves = 4;                  // wavefronts per workgroup
-
 // two neighbouring levels of a row, on any 8-byte boundary
 typedef double les2 __attribute__((ext_vector_type(2)));
 typedef les2 les2u __attribute__((aligned(8)));
 
-// Interior columns: two neighbouring levels per lane, a wavefront per chunk of
-// a column, bin after bin, the next bin's rows (number, every mass species,
-// their tendencies) loaded before the current one's are stored.  Per row: the
-// tendency floored and added, the bottom and top levels from their two
-// neighbours (read lane to lane, before the clamps), the clamp, the new value
-// and a zero tendency stored, at an edge also to the periodic images; per bin
-// the diagnostic sums in bin order and whether any removal test of les_remove
-// can hold on the clamped values (its conditions as it meets them on values
-// nothing has changed yet, with a margin where they are formed otherwise: false
-// means that it would leave the cell as it is).  MS: the mass rows of an ice
-// bin, one more than a liquid bin has.
+// Interior columns: two neighbouring levels per lane, a workgroup per chunk of
+// a column and in it a wavefront per category, bin after bin, the next bin's
+// rows (number, every mass species, their tendencies) loaded before the current
+// one's are stored.  Per row: the tendency floored and added, the bottom and
+// top levels from their two neighbours (read lane to lane, before the clamps),
+// the clamp, the new value and a zero tendency stored, at an edge also to the
+// periodic images; per bin the diagnostic sums in bin order and whether any
+// removal test of les_remove can hold on the clamped values (its conditions as
+// it meets them on values nothing has changed yet, with a margin where they are
+// formed otherwise: false means that it would leave the cell as it is).  The
+// first wavefront writes the sums and lists the cells.  MS: the mass rows of an
+// ice bin, one more than a liquid bin has.
 //
 // HBM-bound: 32 B per element, each row touched once (1.42 GB at 64 x 64 x 120
-// cells, 338 us, 4.2 TB/s; as passes for the update, the bottom and top rows
-// and halos, the sums and the removals 212 + 48 + 132 + 65 us).  The loop body has no
-// branch around a load or store (lanes past the chunk, and the last of an odd
-// one, repeat its last two levels; edge columns take another copy of the loop):
-// a wait then leaves the stores behind it in flight, which a count that differs
-// by path would not.  Two levels per lane halve the changes of row, each of
-// which is another page.
+// cells, 352 us; as passes for the update, the bottom and top rows and
+// halos, the sums and the removals 212 + 48 + 132 + 65 us).  The loop body has
+// no branch around a load or store (lanes past the chunk, and the last of an
+// odd one, repeat its last two levels; edge columns take another copy of the
+// loop): a wait then leaves the stores behind it in flight, which a count that
+// differs by path would not.  Two levels per lane halve the changes of row, each
+// of which is another page.  On small grids the chain of bins sets the time: by
+// category it has 11 links, with one wavefront for all categories 26 (a call on
+// 2 000 cells 82 us, with one wavefront 111, as passes 89; the large grid 389,
+// 375 and 486).
 template <int MS>
-__global__ void __launch_bounds__(64 * kLesWaves) k_les_cells(LesArgs a) {
-  const int ncat = a.level == 5 ? 4 : 3;
+__global__ void __launch_bounds__(256) k_les_cells(LesArgs a) {
+  __shared__ les2 sum[6][64];                 // rc's two parts, sp, sn, si, sr
+  __shared__ int hit[64];                     // bit u: the lane's level u may be changed
   constexpr int iwa = MS - 2, irim = MS - 1, nwet = MS - 1, ndry = MS - 2;
   const int64_t n3 = a.n3;
   const int nx = a.nxp - 4, ny = a.nyp - 4, nch = les_chunks(a.nzp);
   const int lane = threadIdx.x & 63;
-  const int unit = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kLesWaves + threadIdx.x / 64));
-  if (unit >= nx * ny * nch) return;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), unit = (int)blockIdx.x;
+  if (wv == 0) hit[lane] = 0;
+  __syncthreads();
   // the rows of columns at the y edges first: they have the most images
   const int q = unit / nch, h = unit % nch, i = 2 + q % nx, j = 2 + (q / nx + ny - 2) % ny;
   const int k0 = (int)((int64_t)h * a.nzp / nch), nlev = (int)((int64_t)(h + 1) * a.nzp / nch) - k0;
@@ -375,7 +379,7 @@ __global__ void __launch_bounds__(64 * kLesWaves) k_les_cells(LesArgs a) {
     return o;
   };
   bool any[2] = {false, false};
-  les2 sa = zero, sc = zero, sp = zero, sn = zero, si = zero, sr = zero;
+  les2 s1 = zero, s2 = zero;                  // the category's sums: water, and precipitation's number or ice's rime
   struct Bin { les2 n, nt, m[MS], mt[MS]; };
   // bin b of category c
   auto load = [&](int c, int b, Bin &B) {
@@ -393,15 +397,12 @@ __global__ void __launch_bounds__(64 * kLesWaves) k_les_cells(LesArgs a) {
   };
   auto run = [&](auto edge) {
     Bin B, F;
-    // category c is a constant, so that every sum stays in its register
     auto category = [&](auto cc) {
       constexpr int c = decltype(cc)::value;
       const int nb = a.nb[c], nsw = MS - 1 + (c == 3);
+      if (nb > 0) load(c, 0, B);
       for (int b = 0; b < nb; ++b) {
-        const bool more = b + 1 < nb;
-        int cn = more ? c : c + 1;
-        while (cn < ncat && cn != c && a.nb[cn] == 0) ++cn;
-        load(cn < ncat ? cn : c, cn < ncat ? (more ? b + 1 : 0) : b, F);
+        load(c, b + 1 < nb ? b + 1 : b, F);
         const les2 n2 = fresh(B.n, B.nt);
         les2 m2[MS];
 #pragma unroll
@@ -457,38 +458,42 @@ __global__ void __launch_bounds__(64 * kLesWaves) k_les_cells(LesArgs a) {
           }
         }
         if constexpr (c == 0) {
-          if (b >= a.in1a && b <= a.fn2b) sa = sa + wv;
+          if (b >= a.in1a && b <= a.fn2b) s1 = s1 + wv;
         } else if constexpr (c == 1) {
-          if (b >= a.ica_cur && b <= a.fcb_cur) sc = sc + wv;
-        } else if constexpr (c == 2) {
-          sp = sp + wv;
-          sn = sn + n2;
+          if (b >= a.ica_cur && b <= a.fcb_cur) s1 = s1 + wv;
         } else {
-          si = si + wv;
-          sr = sr + rv;
+          s1 = s1 + wv;
+          s2 = s2 + (c == 2 ? n2 : rv);
         }
         B = F;
       }
     };
-    int c0 = 0;
-    while (c0 < ncat - 1 && a.nb[c0] == 0) ++c0;
-    load(c0, 0, B);
-    category(std::integral_constant<int, 0>{});
-    category(std::integral_constant<int, 1>{});
-    category(std::integral_constant<int, 2>{});
-    if (ncat == 4) category(std::integral_constant<int, 3>{});
+    if (wv == 0) category(std::integral_constant<int, 0>{});
+    else if (wv == 1) category(std::integral_constant<int, 1>{});
+    else if (wv == 2) category(std::integral_constant<int, 2>{});
+    else category(std::integral_constant<int, 3>{});
   };
   if (im) run(std::true_type{});
   else run(std::false_type{});
+  if (wv) {
+    sum[wv < 2 ? 1 : 2 * wv - 2][lane] = s1;
+    if (wv >= 2) sum[2 * wv - 1][lane] = s2;
+    if (any[0] || any[1]) atomicOr(hit + lane, (any[0] ? 1 : 0) | (any[1] ? 2 : 0));
+  }
+  __syncthreads();
+  if (wv) return;
+  any[0] |= hit[lane] & 1;
+  any[1] |= (hit[lane] >> 1) & 1;
   // diagnostic tracers (:370-400), as les_sums forms them
   {
-    const les2 rc = sa + sc;
+    const les2 rc = s1 + sum[1][lane], sp = sum[2][lane], sn = sum[3][lane];
     auto sums = [&](int64_t y) {
       les2 rtot = rc + sp + get(a.rp + y);
       set(a.diag + y, rc);
       set(a.diag + n3 + y, sp);
       set(a.diag + 2 * n3 + y, sn);
       if (a.level == 5) {
+        const les2 si = sum[4][lane], sr = sum[5][lane];
         rtot = rtot + si + sr;
         set(a.diag + 4 * n3 + y, si);
         set(a.diag + 5 * n3 + y, sr);
@@ -611,7 +616,7 @@ int launch_les_update(const LesArgs &a, hipStream_t s) {
       a.nwet != ms - 1 || a.ndry != ms - 2 || a.iwa != ms - 2 || (ncat == 4 && a.irim != ms - 1))
     return (int)hipErrorInvalidValue;
   const int64_t units = (int64_t)(a.nxp - 4) * (a.nyp - 4) * les_chunks(a.nzp);
-  const dim3 gc((unsigned)((units + kLesWaves - 1) / kLesWaves)), tc(64 * kLesWaves);
+  const dim3 gc((unsigned)units), tc(64 * ncat);
   if (ms == 3) hipLaunchKernelGGL(k_les_cells<3>, gc, tc, 0, s, a);
   else hipLaunchKernelGGL(k_les_cells<4>, gc, tc, 0, s, a);
   if (nrow <= kLesLdsRows) {
