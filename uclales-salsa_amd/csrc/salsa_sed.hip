@@ -41,23 +41,41 @@ namespace salsa {
 namespace {
 
 constexpr int kSedMaxZ = 256;                 // levels per column (SedArgs::dzt)
+constexpr int kSedSpec = 3;                   // mass rows of a liquid bin that a context holds; ice has one more
 constexpr double kPiFull = 3.14159265358979323846, kKb = 1.3807e-23, kG = 9.81, kCp = 1005., kAlvl = 2.5e6;
 constexpr double kLn10 = 2.302585092994045684;
 
-__device__ double sd_terminal_vel(double diam, double rhop, double rhoa, double visc, double beta) {
-  if (diam <= 19e-6) return (diam * diam) * (rhop - rhoa) * kGrav * beta / (18. * visc);
+// Air at one level: viscosity, mean free path, and the quotients that every
+// bin's fall speed takes from them (divisions are the larger part of it).
+struct Air { double avis, lambda, il, iv, nu; };   // il 1 / (2 lambda), iv 1 / avis, nu avis / density
+__device__ __forceinline__ Air sd_air(double tk, double adn) {
+  Air a;
+  const double tr = tk / 296.16;
+  a.avis = 1.8325e-5 * (416.16 / (tk + 120.0)) * (tr * ::sqrt(tr));
+  const double va = ::sqrt(8 * kKb * tk / (kPiFull * 4.8096e-26));
+  a.lambda = 2 * a.avis / (adn * va);
+  a.il = 0.5 / a.lambda;
+  a.iv = 1. / a.avis;
+  a.nu = a.avis / adn;
+  return a;
+}
+
+// rdiam: 1 / diam
+__device__ __forceinline__ double sd_terminal_vel(double diam, double rdiam, double rhop, double rhoa, const Air &air,
+                                                  double beta) {
+  if (diam <= 19e-6) return (diam * diam) * (rhop - rhoa) * kGrav * beta * air.iv * (1. / 18.);
   if (diam > 19e-6 && diam < 1.07e-3) {
-    const double NDa = 4. / 3. * (diam * diam * diam) * kGrav * (rhop - rhoa) * rhoa / (visc * visc);
+    const double NDa = 4. / 3. * (diam * diam * diam) * kGrav * (rhop - rhoa) * rhoa * (air.iv * air.iv);
     const double X = ::log(NDa);
     const double X2 = X * X, X3 = X2 * X, X4 = X2 * X2, X5 = X4 * X, X6 = X3 * X3;
     const double Y = -0.318657e1 + 0.992696 * X - 0.153193e-2 * X2 - 0.987059e-3 * X3 - 0.578878e-3 * X4 +
                      0.855176e-4 * X5 - 0.327815e-5 * X6;
     const double Re2 = beta * ::exp(Y);
-    return visc / rhoa / diam * Re2;
+    return air.nu * rdiam * Re2;
   }
   // Np**(1/6) through log(Np) / 6: X3 = log(Bo) + log(Np) / 6 and
   // Re3 = exp(log(Np) / 6 + Y3), within a few 1e-16 of the powers
-  const double v2 = visc * visc;
+  const double v2 = air.avis * air.avis;
   const double Np = (kSurfw0 * kSurfw0 * kSurfw0) * (rhoa * rhoa) / ((v2 * v2) * (rhop - rhoa) * kGrav);
   const double L6 = ::log(Np) / 6.;
   const double Bo = 4. / 3. * (rhop - rhoa) * kGrav / kSurfw0 * (diam * diam);
@@ -66,38 +84,20 @@ __device__ double sd_terminal_vel(double diam, double rhop, double rhoa, double 
   const double Y3 = -0.500015e1 + 0.523778e1 * X3 - 0.204914e1 * Z2 + 0.475294 * Z3 - 0.542819e-1 * Z4 +
                     0.238449e-2 * Z5;
   const double Re3 = ::exp(L6 + Y3);
-  return fmin(visc / rhoa / diam * Re3, 9.2);
+  return fmin(air.nu * rdiam * Re3, 9.2);
 }
 
-struct Air { double avis, lambda; };
-__device__ __forceinline__ Air sd_air(double tk, double adn) {
-  Air a;
-  const double tr = tk / 296.16;
-  a.avis = 1.8325e-5 * (416.16 / (tk + 120.0)) * (tr * ::sqrt(tr));
-  const double va = ::sqrt(8 * kKb * tk / (kPiFull * 4.8096e-26));
-  a.lambda = 2 * a.avis / (adn * va);
-  return a;
-}
-
-// the bin's wet diameter, density, slip correction and fall speed
-// from the bin's volume v = sum m_s / rho_s and mass ms = sum m_s
+// the bin's wet diameter, density, slip correction and fall speed from the
+// bin's number zpn >= 1e-15, volume v = sum m_s / rho_s and mass ms = sum m_s;
+// the density ms / zpn over the volume kPi6 dwet**3 = v / zpn of a particle
 __device__ __forceinline__ double sd_vc_sums(double zpn, double v, double ms, double adn, const Air &air,
                                              double *dwet_out, double *gg_out) {
-  const double dwet = zpn < 1.e-15 ? 0. : cbrt_fast(v / zpn / kPi6);
-  const double zdn = ms / zpn / (kPi6 * (dwet * dwet * dwet));
-  const double Kn = 2. * air.lambda / dwet;
-  const double GG = 1. + Kn * (1.249 + 0.42 * ::exp(-0.87 / Kn));
+  const double dwet = cbrt_fast(div_nr(v, zpn) * (1. / kPi6)), rdwet = rcp_nr(dwet);
+  const double zdn = div_nr(ms, v);
+  const double GG = 1. + 2. * air.lambda * rdwet * (1.249 + 0.42 * ::exp(-0.87 * (dwet * air.il)));
   if (dwet_out) *dwet_out = dwet;
   if (gg_out) *gg_out = GG;
-  return sd_terminal_vel(dwet, zdn, adn, air.avis, GG);
-}
-
-__device__ double sd_vc(const SedArgs &a, double zpn, const double *mb, int64_t mstride, double adn, const Air &air,
-                        double *dwet_out, double *gg_out) {
-  double v = 0., ms = 0.;
-  for (int s = 0; s < a.ns; ++s) v = v + mb[s * mstride] / a.rholiq[s];
-  for (int s = 0; s < a.ns; ++s) ms = ms + mb[s * mstride];
-  return sd_vc_sums(zpn, v, ms, adn, air, dwet_out, gg_out);
+  return sd_terminal_vel(dwet, rdwet, zdn, adn, air, GG);
 }
 
 __device__ __forceinline__ bool sd_interior(const SedArgs &a, int i, int j) {
@@ -196,7 +196,7 @@ __global__ void __launch_bounds__(kSedMaxZ, MS <= 3 ? 3 : 1) k_sed_slow(SedArgs 
       double v = 0., ms = 0.;
 #pragma unroll
       for (int s = 0; s < MS; ++s)
-        if (s < ns) v = v + m[s] / a.rholiq[s];
+        if (s < ns) v = v + m[s] * a.rrholiq[s];
 #pragma unroll
       for (int s = 0; s < MS; ++s)
         if (s < ns) ms = ms + m[s];
@@ -280,7 +280,6 @@ size_t sed_slow_lds_bytes(int Z, int nb, int MS) {
 // getShapeCoefficients, terminal_vel's ice branch), water and rime in the
 // rate, the surface rate and tlt, latent heat alvi; MS: the most mass rows
 // per bin (registers per level).
-constexpr int kSedMaxIce = 16;                // ice bins whose rime changes a workgroup keeps in LDS
 
 // The ice fall speed of one bin (DepositionFast flag 4: calcDiamLES,
 // getShapeCoefficients and getDiameter, mo_ice_shape.f90:47-86, 145-191;
@@ -290,57 +289,67 @@ constexpr int kSedMaxIce = 16;                // ice bins whose rime changes a w
 // Dgr = (alpha / (pi6 rho_b))**(1/(3-beta)), Dcr = Dgr h**(1/(3-beta))),
 // the Best number X = 2 vb (rhop-rhoa) g / (gamma rhoa visc**2) D**(2-sigma)
 // and the speed Are / X**bre * visc**(1-2 bre) * (2 alpha g / (rhoa gamma))**bre
-// * D**bv as one exponential: five logarithms and two exponentials per bin
-// instead of eight powers, within a few 1e-14 of the power form.  lvisc:
-// log(visc) of the level; c: the logs of the constant thresholds.
-struct IceLogC { double lmth, lia, lpi6ic; };
-__device__ inline double ice_vc_log(const SedArgs &a, const IceLogC &c, double dsph, double rhop, double rhoa,
-                                    double visc, double lvisc, double mpri, double mrim, double numc) {
-  const double ia = a.ice_alpha, ib = a.ice_beta;
-  double al = kPi6 * kRhoic, be = 3., ga = kPi / 4., si = 2.;
+// * D**bv as one exponential: four logarithms (five for partly rimed ice) and
+// two exponentials per bin instead of eight powers, within a few 1e-14 of the
+// power form.  numc: the number, v, ms: volume sum m / rho and mass sum m of
+// the bin; lvisc, lrhoa: logarithms of the level's viscosity and density; c:
+// those of the constants.
+struct IceLogC { double lmth, lia, lpi6ic, lga, lpi4, l2g, inv, rib; };   // inv 1 / (3 - beta), rib 1 / beta
+__device__ __forceinline__ double ice_vc_log(const SedArgs &a, const IceLogC &c, double v, double ms, double rhoa,
+                                             double lvisc, double lrhoa, double mpri, double mrim, double numc) {
+  double lal = c.lpi6ic, be = 3., lga = c.lpi4, si = 2.;
   double Ld = -20.72326583694641;               // log(1e-9): getDiameter's value below the number limit
+  const double rn = rcp_nr(numc);
   if (!(numc < 1.e-6)) {
-    const double mtot = (mpri + mrim) / numc;
-    const double fr = fmax(fmin(mrim / (mtot * numc), 0.9999), 0.0001);
+    const double mt = mpri + mrim, mtot = mt * rn;
+    const double fr = fmax(fmin(div_nr(mrim, mt), 0.9999), 0.0001);
     const double rho_b = fr * kRhori + (1. - fr) * kRhoic;
-    const double Lm = ::log(mtot), Lrb = ::log(kPi6 * rho_b), inv = 1. / (3. - ib);
-    const double lmgr = Lrb + 3. * ((c.lia - Lrb) * inv);
-    const double h = 1. / (1. - fr), Lh = ::log(h);
-    const double lmcr = lmgr + 3. * (Lh * inv);
+    const double Lm = ::log(mtot), Lrb = ::log(kPi6 * rho_b);
+    const double lmgr = Lrb + 3. * ((c.lia - Lrb) * c.inv);
+    const double Lh = -::log(1. - fr);
+    const double lmcr = lmgr + 3. * (Lh * c.inv);
     if (Lm >= c.lmth && Lm < lmgr) {
-      al = ia; be = ib; ga = a.ice_gamma; si = a.ice_sigma;
+      lal = c.lia; be = a.ice_beta; lga = c.lga; si = a.ice_sigma;
     } else if (Lm > lmcr) {
-      al = ia * h; be = ib; ga = a.ice_gamma * (1. - fr) + kPi / 4. * fr; si = a.ice_sigma * (1. - fr) + 2. * fr;
+      lal = c.lia + Lh; be = a.ice_beta; si = a.ice_sigma * (1. - fr) + 2. * fr;
+      lga = ::log(a.ice_gamma * (1. - fr) + kPi / 4. * fr);
     }
-    if (Lm < c.lmth) Ld = (Lm - c.lpi6ic) / 3.;
-    else if (Lm < lmgr) Ld = (Lm - c.lia) / ib;
-    else if (Lm < lmcr) Ld = (Lm - Lrb) / 3.;
-    else if (Lm >= lmcr) Ld = (Lm - Lh - c.lia) / ib;
+    if (Lm < c.lmth) Ld = (Lm - c.lpi6ic) * (1. / 3.);
+    else if (Lm < lmgr) Ld = (Lm - c.lia) * c.rib;
+    else if (Lm < lmcr) Ld = (Lm - Lrb) * (1. / 3.);
+    else if (Lm >= lmcr) Ld = (Lm - Lh - c.lia) * c.rib;
   }
   const double c1 = 0.0902, delta0 = 9.06;
-  const double vb = kPi6 * cubed(dsph);
-  const double LX = ::log(2. * vb * (rhop - rhoa) * kGrav / (ga * rhoa * visc * visc)) + (2. - si) * Ld;
-  const double sX = ::sqrt(::exp(LX));
-  const double k1213 = ::sqrt(1. + c1 * sX);
-  const double bre = 0.5 * c1 * sX / (k1213 - 1.) / k1213;
-  const double Lc = ::log((2. * al * kGrav) / (rhoa * ga));
+  const double lgr = lga + lrhoa;
+  const double LX = ::log(2. * kGrav * (v * rn) * (div_nr(ms, v) - rhoa)) - lgr - 2. * lvisc + (2. - si) * Ld;
+  const double sX = ::exp(0.5 * LX);
+  const double k1213 = ::sqrt(1. + c1 * sX), k1 = k1213 - 1.;
+  const double bre = div_nr(0.5 * c1 * sX, k1 * k1213);
   const double bv = bre * (be - si + 2.) - 1.;
-  return 0.25 * delta0 * delta0 * (k1213 - 1.) * (k1213 - 1.) *
-         ::exp(-bre * LX + (1. - 2. * bre) * lvisc + bre * Lc + bv * Ld);
+  return 0.25 * delta0 * delta0 * k1 * k1 *
+         ::exp(-bre * LX + (1. - 2. * bre) * lvisc + bre * (c.l2g + lal - lgr) + bv * Ld);
 }
 
 // LDS of one column (Z = blockDim.x levels), carved from the dynamic buffer
-// in this order: dz, rdz, adn [Z]; vc [2][Z] (source fall speed, by bin
-// parity); c1, c0, q [2][Z] (by quantity parity); rem [ns*nb] (deposited
-// mass per species and bin); rout [nb][Z] (ice: rime change per bin); then
-// the ints dec [2][Z] (bit 0 source, 1 two levels, 2 deposits; (d + 1) << 8)
-// and wmax [2][4] (largest fall distance per wavefront, by bin parity).
-__host__ __device__ inline size_t sed_prc_lds_bytes(int Z, int nb, int ns, bool ice) {
-  return (size_t)(11 * Z + ns * nb + (ice ? nb * Z : 0)) * sizeof(double) + (size_t)(2 * Z + 8) * sizeof(int);
+// in this order: dz, rdz [Z]; by bin parity f1, f0 (shares of a source's
+// content that land one level below kf and on it), av (air density times fall
+// speed) [2][Z] and q (its number and masses) [2][1 + MS][Z]; rem [ns*nb]
+// (deposited mass per species and bin); then the ints dec [2][Z] (bit 0
+// source, 1 two levels, 2 deposits; (d + 1) << 8) and wmax [2][4] (largest
+// fall distance per wavefront).
+__host__ __device__ inline size_t sed_prc_lds_bytes(int Z, int nb, int ns, int MS) {
+  return (size_t)((8 + 2 * (1 + MS)) * Z + ns * nb) * sizeof(double) + (size_t)(2 * Z + 8) * sizeof(int);
 }
 
+// Bound by the fall speed's FP64 arithmetic and, at level 4, HBM.  One barrier
+// per bin: a source publishes its content and the two shares, and every level
+// scans the sources above it once for all quantities.  With a barrier and a
+// scan per bin and moved quantity (35 and 21 of them) and true divisions the
+// ice launch took 925 us at 128 x 128 x 100 cells and the precipitation launch
+// 141 us at 64 x 64 x 120; now 590 and 94 us. (Three wavefronts per SIMD without
+// the few spills of four: the same times; two: a fifth longer.)
 template <int MS, bool ICE>
-__global__ void __launch_bounds__(kSedMaxZ, (MS <= 3 && !ICE) ? 4 : 1) k_sed_prc(SedArgs a) {
+__global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
   extern __shared__ double smem[];
   constexpr int cat = ICE ? 3 : 2;
   constexpr double alv = ICE ? kAls : kAlvl;
@@ -350,10 +359,9 @@ __global__ void __launch_bounds__(kSedMaxZ, (MS <= 3 && !ICE) ? 4 : 1) k_sed_prc
   const int k = threadIdx.x, nzp = a.nzp, ktop = nzp - 2, nw = blockDim.x / 64;
   const int nb = a.nb[cat], ns = ICE ? a.ns_ice : a.ns, iw = a.iwa, ir = a.irim;
   const int Z = blockDim.x;
-  double *const Sdz = smem, *const Srdz = smem + Z, *const Sadn = smem + 2 * Z, *const Svc = smem + 3 * Z;
-  double *const Sc1 = smem + 5 * Z, *const Sc0 = smem + 7 * Z, *const Sq = smem + 9 * Z, *const Srem = smem + 11 * Z;
-  double *const Srout = Srem + ns * nb;
-  int *const Sdec = reinterpret_cast<int *>(Srout + (ICE ? nb * Z : 0));
+  double *const Sdz = smem, *const Srdz = smem + Z, *const Sf1 = smem + 2 * Z, *const Sf0 = smem + 4 * Z;
+  double *const Sav = smem + 6 * Z, *const Sq = smem + 8 * Z, *const Srem = Sq + 2 * (1 + MS) * Z;
+  int *const Sdec = reinterpret_cast<int *>(Srem + ns * nb);
   int *const Swmax = Sdec + 2 * Z;
   const double *__restrict__ Np = a.n_p[cat];
   const double *__restrict__ Mp = a.m_p[cat];
@@ -364,7 +372,7 @@ __global__ void __launch_bounds__(kSedMaxZ, (MS <= 3 && !ICE) ? 4 : 1) k_sed_prc
   double *__restrict__ srate = ICE ? a.sfcirate : a.sfcrrate;
   const bool lev = k < nzp, src = k >= 1 && k <= ktop;
   const int64_t x = col * nzp + k;
-  const double dtlt = a.dtlt;
+  const double dtlt = a.dtlt, rdt = 1. / dtlt;
   // the bin's rows at this level, quantity u: 0 the number, 1 + s species s
   // (the next bin's are loaded while the current one is worked on)
   double qv[MS + 1], tv[MS + 1], qn[MS + 1], tn[MS + 1];
@@ -378,74 +386,72 @@ __global__ void __launch_bounds__(kSedMaxZ, (MS <= 3 && !ICE) ? 4 : 1) k_sed_prc
     }
   };
   load(0, qv, tv);
-  Air air = {0., 0.};
-  double rr = 0., sw = 0.;
-  IceLogC ilc{0., 0., 0.};                      // ice: log Mth (pristine threshold), log alpha, log(pi6 rhoic)
+  Air air = {0., 0., 0., 0., 0.};
+  double rr = 0., sw = 0., sr = 0., ad = 0., lvisc = 0., lrhoa = 0.;
+  IceLogC ilc{0., 0., 0., 0., 0., 0., 0., 0.};          // ice: log Mth (pristine threshold), log alpha, log(pi6 rhoic), ..
   if (ICE) {
     const double dth = ::pow(kPi6 * kRhoic / a.ice_alpha, 1. / (a.ice_beta - 3.));
     ilc.lmth = ::log(kRhoic * kPi6 * cubed(dth));
     ilc.lia = ::log(a.ice_alpha);
     ilc.lpi6ic = ::log(kPi6 * kRhoic);
+    ilc.lga = ::log(a.ice_gamma);
+    ilc.lpi4 = ::log(kPi / 4.);
+    ilc.l2g = ::log(2. * kGrav);
+    ilc.inv = 1. / (3. - a.ice_beta);
+    ilc.rib = 1. / a.ice_beta;
   }
-  double lvisc = 0.;
   if (lev) {
     Sdz[k] = a.dzt[k];
     Srdz[k] = 1. / a.dzt[k];
-    Sadn[k] = a.adn[x];
+    ad = a.adn[x];
   }
   if (src) {
-    air = sd_air(a.tk[x], a.adn[x]);
-    if (ICE) lvisc = ::log(air.avis);
+    air = sd_air(a.tk[x], ad);
+    if (ICE) {
+      lvisc = ::log(air.avis);
+      lrhoa = ::log(ad);
+    }
     rr = rate[x];
   }
   __syncthreads();
   for (int b = 0; b < nb; ++b) {
     const int pb = b & 1;
+    double *const Q = Sq + pb * (1 + MS) * Z;
     load(b + 1, qn, tn);
     const double zpn = qv[0];
     const bool on = src && !(zpn < kPrlim);
-    double vc = 0., pre = 0., dA = 0., dB = 0.;
+    double f1 = 0., f0 = 0.;
     int d = -1;
     bool two = false, dep = false;
     if (on) {
-      if (ICE) {
-        // calcDiamLES (mo_particle_external_properties.f90:169-201) both
-        // ways, getShapeCoefficients, the bulk density, terminal_vel flag 4
-        double v = 0., mpri = 0., ms = 0., mrim = 0.;
+      double v = 0., ms = 0., vc, wv = 0., rv = 0.;
 #pragma unroll
-        for (int s = 0; s < MS; ++s)
-          if (s < ns) v = v + qv[1 + s] / a.rhoice[s];
-#pragma unroll
-        for (int s = 0; s < MS; ++s)
-          if (s < ns - 1) mpri = mpri + qv[1 + s];
-#pragma unroll
-        for (int s = 0; s < MS; ++s)
-          if (s == ns - 1) mrim = qv[1 + s];
-        const double dwet = zpn < 1.e-15 ? 0. : cbrt_fast(v / zpn / kPi6);
-#pragma unroll
-        for (int s = 0; s < MS; ++s)
-          if (s < ns) ms = ms + qv[1 + s];
-        const double zdn = ms / zpn / (kPi6 * (dwet * dwet * dwet));
-        vc = ice_vc_log(a, ilc, dwet, zdn, Sadn[k], air.avis, lvisc, mpri, mrim, zpn);
-      } else {
-        double v = 0., ms = 0.;
-#pragma unroll
-        for (int s = 0; s < MS; ++s)
-          if (s < ns) v = v + qv[1 + s] / a.rholiq[s];
-#pragma unroll
-        for (int s = 0; s < MS; ++s)
-          if (s < ns) ms = ms + qv[1 + s];
-        vc = sd_vc_sums(zpn, v, ms, Sadn[k], air, nullptr, nullptr);
-      }
-      vt[(int64_t)b * n3 + x] = vc;
-      // the rate: water (and, for ice, rime) falling out of the level (:1206-1212)
-      double wv = 0., rv = 0.;
+      for (int s = 0; s < MS; ++s)
+        if (s < ns) {
+          v = v + qv[1 + s] * (ICE ? a.rrhoice : a.rrholiq)[s];
+          ms = ms + qv[1 + s];
+        }
 #pragma unroll
       for (int s = 0; s < MS; ++s) {
         if (s == iw) wv = qv[1 + s];
         if (s == ir) rv = qv[1 + s];
       }
-      rr = ICE ? rr + (wv + rv) * Sadn[k] * vc * alv : rr + wv * Sadn[k] * vc * alv;
+      if (ICE) {
+        // calcDiamLES (mo_particle_external_properties.f90:169-201) both
+        // ways, getShapeCoefficients, the bulk density, terminal_vel flag 4
+        double mpri = 0., mrim = 0.;
+#pragma unroll
+        for (int s = 0; s < MS; ++s) {
+          if (s < ns - 1) mpri = mpri + qv[1 + s];
+          if (s == ns - 1) mrim = qv[1 + s];
+        }
+        vc = ice_vc_log(a, ilc, v, ms, ad, lvisc, lrhoa, mpri, mrim, zpn);
+      } else {
+        vc = sd_vc_sums(zpn, v, ms, ad, air, nullptr, nullptr);
+      }
+      vt[(int64_t)b * n3 + x] = vc;
+      // the rate: water (and, for ice, rime) falling out of the level (:1206-1212)
+      rr = ICE ? rr + (wv + rv) * ad * vc * alv : rr + wv * ad * vc * alv;
       const double fdmax = dtlt * vc;
       double fd = 0.;
       int fi = 0;
@@ -458,66 +464,69 @@ __global__ void __launch_bounds__(kSedMaxZ, (MS <= 3 && !ICE) ? 4 : 1) k_sed_prc
       const int kf = k - fi;                    // kf - 1 >= 0; kf <= k + 1 <= nzp - 1
       fd = fd - Srdz[kf];
       const double fdos = fmin(fmax(fdmax - fd, 0.), Srdz[kf]);
-      pre = fdos * Sdz[kf];
+      const double pre = fdos * Sdz[kf];
       two = !(pre > 0.5);
-      dA = Sdz[kf - 1];
-      dB = two ? Sdz[kf] : Sdz[k];
+      // the shares (:1229-1246), thinner or thicker levels included
+      f1 = (two ? pre : 1.) * Sdz[kf - 1] * Srdz[two ? kf : k];
+      f0 = two ? 1. - pre : 0.;
       d = k - kf;                               // >= -1
-      Svc[pb * Z + k] = vc;
+      Sf1[pb * Z + k] = f1;
+      Sf0[pb * Z + k] = f0;
+      Sav[pb * Z + k] = ad * vc;
+#pragma unroll
+      for (int u = 0; u <= MS; ++u) Q[u * Z + k] = qv[u];
     }
     Sdec[pb * Z + k] = on ? (1 | (two ? 2 : 0) | (dep ? 4 : 0) | ((d + 1) << 8)) : 0;
     int wm = d;
     for (int o = 32; o > 0; o >>= 1) wm = max(wm, __shfl_xor(wm, o));
     if ((k & 63) == 0) Swmax[pb * 4 + (k >> 6)] = wm;
+    __syncthreads();
     int dmax = -1;
+    for (int w = 0; w < nw; ++w) dmax = max(dmax, Swmax[pb * 4 + w]);
+    double out[MS + 1];
 #pragma unroll
-    for (int qy = 0; qy <= MS; ++qy) {
-      if (qy > ns) break;
-      const int p = (b * (ns + 1) + qy) & 1;    // parity of the c1 / c0 / q buffers
-      const double q = qv[qy];
-      double c1 = 0., c0 = 0.;
+    for (int u = 0; u <= MS; ++u) out[u] = 0.;
+    if (lev && k <= ktop) {
+      // what lands here, from the top down as the reference adds it
+      for (int s = min(ktop, k + dmax + 1); s > k; --s) {
+        const int ds = Sdec[pb * Z + s], kf = s - ((ds >> 8) - 1);
+        const bool l1 = kf - 1 == k, l0 = (ds & 2) && kf == k;
+        if (!(ds & 1) || !(l1 || l0)) continue;
+        const double f = l1 ? Sf1[pb * Z + s] : Sf0[pb * Z + s];
+#pragma unroll
+        for (int u = 0; u <= MS; ++u) out[u] = out[u] + f * Q[u * Z + s];
+      }
       if (on) {
-        // the reference's expressions, left to right (:1229-1246)
-        if (two) {
-          c1 = pre * q * dA / dB;
-          c0 = (1. - pre) * q;
-        } else {
-          c1 = q * dA / dB;
+        // what leaves, and what does not leave the level
+        const double own = d == -1 ? f1 : (two && d == 0 ? f0 : 0.);
+#pragma unroll
+        for (int u = 0; u <= MS; ++u) {
+          out[u] = out[u] - qv[u];
+          if (d <= 0) out[u] = out[u] + own * qv[u];
         }
-        Sc1[p * Z + k] = c1;
-        Sc0[p * Z + k] = c0;
-        if (dep) Sq[p * Z + k] = q;
       }
-      __syncthreads();
-      if (qy == 0)
-        for (int w = 0; w < nw; ++w) dmax = max(dmax, Swmax[pb * 4 + (w)]);
-      if (lev) {
-        double out = 0.;
-        if (k <= ktop) {
-          for (int s = min(ktop, k + dmax + 1); s > k; --s) {
-            const int ds = Sdec[pb * Z + s];
-            if (!(ds & 1)) continue;
-            const int kf = s - ((ds >> 8) - 1);
-            if (kf - 1 == k) out = out + Sc1[p * Z + s];
-            if ((ds & 2) && kf == k) out = out + Sc0[p * Z + s];
-          }
-          if (on) {
-            out = out - q;
-            if (d == -1) out = out + c1;        // particles that do not leave the level
-            if (two && d == 0) out = out + c0;
-          }
-        }
-        const int64_t r = qy == 0 ? (int64_t)b * n3 : ((int64_t)(qy - 1) * nb + b) * n3;
-        (qy == 0 ? Nt : Mt)[r + x] = tv[qy] + out / dtlt;
-        if (qy - 1 == iw) sw = sw + out;
-        if (ICE && qy - 1 == ir) Srout[b * Z + k] = out;
+    }
+    if (lev) {
+#pragma unroll
+      for (int u = 0; u <= MS; ++u) {
+        if (u > ns) break;
+        const int64_t r = u == 0 ? (int64_t)b * n3 : ((int64_t)(u - 1) * nb + b) * n3;
+        (u == 0 ? Nt : Mt)[r + x] = tv[u] + out[u] * rdt;
+        if (u - 1 == iw) sw = sw + out[u];
+        if (ICE && u - 1 == ir) sr = sr + out[u];
       }
-      if (qy > 0 && k == 0) {                   // lane 0 (level 0 is never a source)
-        double r = 0.;
-        for (int s = min(ktop, dmax + 1); s >= 1; --s)
-          if ((Sdec[pb * Z + s] & 5) == 5) r = r + Sq[p * Z + s] * Sadn[s] * Svc[pb * Z + s];
-        Srem[(qy - 1) * nb + b] = r;
-      }
+    }
+    if (k == 0) {                               // lane 0 (level 0 is never a source)
+      double r[MS];
+#pragma unroll
+      for (int s = 0; s < MS; ++s) r[s] = 0.;
+      for (int s = min(ktop, dmax + 1); s >= 1; --s)
+        if ((Sdec[pb * Z + s] & 5) == 5)
+#pragma unroll
+          for (int u = 0; u < MS; ++u) r[u] = r[u] + Q[(1 + u) * Z + s] * Sav[pb * Z + s];
+#pragma unroll
+      for (int u = 0; u < MS; ++u)
+        if (u < ns) Srem[u * nb + b] = r[u];
     }
 #pragma unroll
     for (int u = 0; u <= MS; ++u) {
@@ -526,12 +535,8 @@ __global__ void __launch_bounds__(kSedMaxZ, (MS <= 3 && !ICE) ? 4 : 1) k_sed_prc
     }
   }
   if (src) rate[x] = rr;
-  if (lev && k <= ktop) {
-    // SUM over the water rows in bin order, for ice then the rime rows
-    if (ICE)
-      for (int b = 0; b < nb; ++b) sw = sw + Srout[b * Z + k];
-    a.tlt[x] = a.tlt[x] - (sw / dtlt) * (alv / kCp) * a.th[x] / a.tk[x];
-  }
+  // the water rows and, for ice, the rime rows
+  if (lev && k <= ktop) a.tlt[x] = a.tlt[x] - ((sw + sr) * rdt) * (alv / kCp) * a.th[x] / a.tk[x];
   if (k == 0) {
     // SUM(remprc((ns-1)*nb:ns*nb)) (ice: (ns-2)*nb:ns*nb), 1-based, one entry
     // before the water rows as written (:1256-1260)
@@ -551,38 +556,22 @@ int launch_sedim(const SedArgs &a, int sed_aero, int sed_cloud, int sed_precp, i
     // one workgroup per interior column, one lane per level; the fluxes of
     // one bin and the column's rain-rate terms in LDS
     const unsigned ncol = (unsigned)((a.nxp - 4) * (a.nyp - 4)), nthr = (unsigned)((a.nzp + 63) / 64 * 64);
-    const int ms = a.ns <= 3 ? 3 : a.ns <= 5 ? 5 : kMaxSpec;
-    const size_t lds = sed_slow_lds_bytes((int)nthr, a.nb[cat], ms);
-    if (a.nzp > kSedMaxZ || a.nb[cat] > 64 || a.ns < 2 || lds > 65536) return (int)hipErrorInvalidValue;
-    if (ms == 3)
-      hipLaunchKernelGGL(k_sed_slow<3>, dim3(ncol), dim3(nthr), lds, s, a, cat);
-    else if (ms == 5)
-      hipLaunchKernelGGL(k_sed_slow<5>, dim3(ncol), dim3(nthr), lds, s, a, cat);
-    else
-      hipLaunchKernelGGL(k_sed_slow<kMaxSpec>, dim3(ncol), dim3(nthr), lds, s, a, cat);
+    const size_t lds = sed_slow_lds_bytes((int)nthr, a.nb[cat], kSedSpec);
+    if (a.nzp > kSedMaxZ || a.nb[cat] > 64 || a.ns < 2 || a.ns > kSedSpec || lds > 65536) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_sed_slow<kSedSpec>, dim3(ncol), dim3(nthr), lds, s, a, cat);
   }
   if (sed_precp) {
     // one workgroup per interior column, one lane per level
     const unsigned ncol = (unsigned)((a.nxp - 4) * (a.nyp - 4)), nthr = (unsigned)((a.nzp + 63) / 64 * 64);
-    const size_t lds = sed_prc_lds_bytes((int)nthr, a.nb[2], a.ns, false);
-    if (a.nzp > kSedMaxZ || lds > 65536) return (int)hipErrorInvalidValue;
-    if (a.ns <= 3)
-      hipLaunchKernelGGL((k_sed_prc<3, false>), dim3(ncol), dim3(nthr), lds, s, a);
-    else if (a.ns <= 5)
-      hipLaunchKernelGGL((k_sed_prc<5, false>), dim3(ncol), dim3(nthr), lds, s, a);
-    else
-      hipLaunchKernelGGL((k_sed_prc<kMaxSpec, false>), dim3(ncol), dim3(nthr), lds, s, a);
+    const size_t lds = sed_prc_lds_bytes((int)nthr, a.nb[2], a.ns, kSedSpec);
+    if (a.nzp > kSedMaxZ || a.ns > kSedSpec || lds > 65536) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_sed_prc<kSedSpec, false>), dim3(ncol), dim3(nthr), lds, s, a);
   }
   if (sed_ice && a.level == 5) {
     const unsigned ncol = (unsigned)((a.nxp - 4) * (a.nyp - 4)), nthr = (unsigned)((a.nzp + 63) / 64 * 64);
-    const size_t lds = sed_prc_lds_bytes((int)nthr, a.nb[3], a.ns_ice, true);
-    if (a.nzp > kSedMaxZ || a.nb[3] > kSedMaxIce || lds > 65536) return (int)hipErrorInvalidValue;
-    if (a.ns_ice <= 3)
-      hipLaunchKernelGGL((k_sed_prc<3, true>), dim3(ncol), dim3(nthr), lds, s, a);
-    else if (a.ns_ice <= 5)
-      hipLaunchKernelGGL((k_sed_prc<5, true>), dim3(ncol), dim3(nthr), lds, s, a);
-    else
-      hipLaunchKernelGGL((k_sed_prc<kMaxSpec, true>), dim3(ncol), dim3(nthr), lds, s, a);
+    const size_t lds = sed_prc_lds_bytes((int)nthr, a.nb[3], a.ns_ice, kSedSpec + 1);
+    if (a.nzp > kSedMaxZ || a.ns_ice > kSedSpec + 1 || lds > 65536) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_sed_prc<kSedSpec + 1, true>), dim3(ncol), dim3(nthr), lds, s, a);
   }
   return (int)hipGetLastError();
 }
