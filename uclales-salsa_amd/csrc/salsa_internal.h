@@ -191,7 +191,9 @@ struct LanesArgs {
   void *K;                            // kernels [block][pair][64], a row of zeros last
   uint8_t *pf;                        // COUNT(D_new > precpbins) per cloud-cloud pair [block][ncc][64]
   double *dwa;                        // wet diameters of the aerosol bins before the step [block][nbins][64]
-  size_t o_pf, o_dwa, o_rows, o_prog;   // byte offsets in the work space
+  void *Ka;                           // K and dwa of the cells without hydrometeors
+  double *dwaa;
+  size_t o_Ka, o_pf, o_dwa, o_dwaa, o_rows, o_prog;   // byte offsets in the work space
 };
 
 // Arguments of the forward-mode derivative kernel: the trajectory starts from

@@ -1168,9 +1168,11 @@ size_t lanes_work(const DevLayout &L, int kt, int64_t ncells, LanesArgs &w) {
   w.gn_aero = (int)(sa / kL);
   size_t o = 0;
   auto take = [&](size_t n) { const size_t at = o; o += (n + 255) / 256 * 256; return at; };
-  take((size_t)(sh * (L.npair + 1) > sa * (L.npair_aa + 1) ? sh * (L.npair + 1) : sa * (L.npair_aa + 1)) * kt);
+  take((size_t)sh * (L.npair + 1) * kt);
+  w.o_Ka = take((size_t)sa * (L.npair_aa + 1) * kt);
   w.o_pf = take((size_t)sh * (L.ncc > 0 ? L.ncc : 1));
-  w.o_dwa = take((size_t)sa * L.nb[0] * 8);
+  w.o_dwa = take((size_t)sh * L.nb[0] * 8);
+  w.o_dwaa = take((size_t)sa * L.nb[0] * 8);
   w.o_rows = take((size_t)L.nt * (1 + lanes_volumes(L)) * sizeof(LaneRow));
   w.o_prog = take((size_t)lanes_program(L, nullptr) * sizeof(uint32_t));
   return o;
@@ -1188,7 +1190,11 @@ int launch_lanes(const DevLayout &L, int precision, bool hyd, const DevLayout *d
                  hipStream_t s) {
   LanesArgs w = w0;
   const int NV = lanes_volumes(L);
-  if (!hyd) w.prog += sweep_program(L, true, nullptr);
+  if (!hyd) {
+    w.prog += sweep_program(L, true, nullptr);
+    w.K = w.Ka;
+    w.dwa = w.dwaa;
+  }
 #define SALSA_LANES(KT, NV_, L5, WP, W, VL, NR)                                                        \
   return hyd ? launch_pair_sweep<KT, NV_, L5, WP, 32, W, VL, NR, true>(L, d, a, w, s)                  \
              : launch_pair_sweep<KT, NV_, L5, 4, kL, kWavesA, kPartA, kBinsA, false>(L, d, a, w, s)
