@@ -1125,8 +1125,8 @@ int sweep_program(const DevLayout &L, bool hyd, uint32_t *prog) {
 }  // namespace
 
 // Slots whose kernels the work space holds: of the cells with hydrometeors,
-// and of those without (fewer pairs).  About 200 MB of FP32 kernels of the
-// 26-bin layout at either size.
+// and of those without (fewer pairs).  About 200 MB of FP32 kernels each of
+// the 26-bin layout.  (Times below: the two lists one after the other.)
 constexpr int kSlotsHyd = 1 << 17, kSlotsAero = 1 << 19;
 
 // The fewest cells of a context that steps with one lane per cell.  A
