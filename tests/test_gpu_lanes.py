@@ -1,6 +1,6 @@
 """The step with one lane per cell (the large grids' path) against the general
 step kernel, which a chosen launch shape selects (16 lanes per cell: the order
-of the sums that the path keeps at level 5): every layout and precision
+of the sums that the mixed path keeps at level 5, FP64 that of 32): every layout and precision
 it takes, grids at the smallest size it runs at and with ragged last
 workgroups, lists that are empty, one short of a workgroup, full and one over,
 tendency and in-place calls, contents below the limits, one NaN cell.

@@ -33,7 +33,7 @@ int launch_act_cloud_base(const DevLayout *d, const StepArgs &a, hipStream_t s);
 int64_t lanes_least(const DevLayout &L);
 bool lanes_fit(const DevLayout &L, int kt, int64_t ncells);
 size_t lanes_work(const DevLayout &L, int kt, int64_t ncells, LanesArgs &w);
-int lanes_program(const DevLayout &L, uint32_t *prog);
+int lanes_program(const DevLayout &L, int kt, uint32_t *prog);
 int launch_lanes_class(const DevLayout &L, const DevLayout *d, const StepArgs &a, const LanesArgs &w, hipStream_t s);
 int launch_lanes(const DevLayout &L, int precision, bool hyd, const DevLayout *d, const StepArgs &a, const LanesArgs &w,
                  hipStream_t s);
@@ -324,8 +324,8 @@ extern "C" int salsa_ctx_create(const salsa_bin_desc *desc, const salsa_params *
       set_error("hipStreamCreate failed");
       return fail(SALSA_ERR_HIP);
     }
-    std::vector<uint32_t> prog((size_t)lanes_program(c->hostL, nullptr));
-    (void)lanes_program(c->hostL, prog.data());
+    std::vector<uint32_t> prog((size_t)lanes_program(c->hostL, kt, nullptr));
+    (void)lanes_program(c->hostL, kt, prog.data());
     if (hipMemcpy(c->lanes_buf + c->lw.o_prog, prog.data(), prog.size() * sizeof(uint32_t), hipMemcpyHostToDevice) !=
         hipSuccess) {
       set_error("copy of the sweep program failed");

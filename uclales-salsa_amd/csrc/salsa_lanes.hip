@@ -45,7 +45,7 @@
 
 namespace salsa {
 
-int lanes_program(const DevLayout &L, uint32_t *prog);
+int lanes_program(const DevLayout &L, int kt, uint32_t *prog);
 
 namespace {
 
@@ -60,7 +60,7 @@ constexpr int kProgT = 8, kProgK = 9, kProgN = 10, kProgS = 12, kProgQ = 13;   /
 constexpr int kProgF = 16;                    // words 16..: precipitation-formation entries:
                                               // pair | bin << 16 | own series << 30 | used << 31
 constexpr int kProg = 32;
-__host__ __device__ constexpr int prog_pf(int VL) { return VL == 16 ? 12 : 8; }   // at most 8, and 3 to align them
+__host__ __device__ constexpr int prog_pf(int VL) { return VL >= 16 ? 12 : 8; }   // at most 8, and 3 to align them
 enum : uint32_t {
   SR_SINK = 1u, SR_SRC = 2u, SR_SINK_EAGG = 4u, SR_SRC_EAGG = 8u, SR_PC_WA = 16u, SR_PC_RI = 32u, SR_PF = 64u,
   SR_FIX_OWN = 128u, SR_FIX_OTH = 256u, SR_SPECIAL = 511u & ~3u
@@ -347,8 +347,8 @@ __device__ __forceinline__ double equil_bin(double n, double zcore, double c1, d
 // Sums over a cell's collectors are taken in VL partial sums, entry e in
 // partial e % VL, which are then added as a balanced tree; a wavefront holds
 // VL / W neighbouring partials and adds them before the W wavefronts' sums
-// meet.  With VL = 16 that is the order of the general kernel's 16 lanes per
-// cell, bit for bit.
+// meet.  With VL = 16 or 32 that is the order of the general kernel's 16 or 32
+// lanes per cell, bit for bit.
 template <int W>
 __device__ __forceinline__ double tree_sum(const double *p, int stride) {
   static_assert(W == 4 || W == 8 || W == 16, "wavefronts per workgroup");
@@ -363,9 +363,10 @@ __device__ __forceinline__ double tree_sum(const double *p, int stride) {
 // the same over the V values of each of a cell's VL / V lanes
 template <int VL, int V>
 __device__ __forceinline__ double tree_lanes(const double (&x)[V]) {
-  static_assert(V == 1 || V == 2, "partials per lane");
+  static_assert(V == 1 || V == 2 || V == 4, "partials per lane");
   if constexpr (V == 1) return cell_sum<VL>(x[0]);
-  else return cell_sum<VL / 2>(x[0] + x[1]);
+  else if constexpr (V == 2) return cell_sum<VL / 2>(x[0] + x[1]);
+  else return cell_sum<VL / 4>((x[0] + x[1]) + (x[2] + x[3]));
 }
 
 // LDS of k_lanes_sweep for nb bins of NV volumes, nice of them ice, and ncc
@@ -585,10 +586,15 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
       for (int q = 0; q < NC; ++q) {
         double y = part[0][q];
         if constexpr (A == 2) y = y + part[1][q];
+        if constexpr (A == 4) y = (y + part[1][q]) + (part[2][q] + part[3][q]);
         p[q * kL] = y;
       }
       if (HYD && (fl & TF_PF)) {
         if constexpr (A == 2) { so[0] = so[0] + so[1]; sx[0] = sx[0] + sx[1]; }
+        if constexpr (A == 4) {
+          so[0] = (so[0] + so[1]) + (so[2] + so[3]);
+          sx[0] = (sx[0] + sx[1]) + (sx[2] + sx[3]);
+        }
         p[(NP - 2) * kL] = so[0];
         p[(NP - 1) * kL] = sx[0];
       }
@@ -721,7 +727,8 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
         }
         y[v / 4] = (z[0] + z[1]) + (z[2] + z[3]);
       }
-      if constexpr (VL == 16) return (y[0] + y[1]) + (y[2] + y[3]);
+      if constexpr (VL == 32) return ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
+      else if constexpr (VL == 16) return (y[0] + y[1]) + (y[2] + y[3]);
       else if constexpr (VL == 8) return y[0] + y[1];
       else return y[0];
     };
@@ -1066,6 +1073,9 @@ constexpr int kMaxLds = 160 * 1024;
 constexpr int kWavesA = 4, kPartA = 4, kBinsA = 12 / 4;
 constexpr int kWaves2 = 4, kPart2 = 4, kBins2 = 24 / 4;
 constexpr int kWaves4 = 8, kPart4 = 16, kBins4 = 2;
+// level 5 in FP64: the order of 32 lanes per cell, at which the general kernel
+// runs there (see tree_sum)
+constexpr int kPart5d = 32, kBins5d = 1;
 
 inline int lanes_volumes(const DevLayout &L) { return L.level == 5 ? L.nspec : L.nwet; }
 
@@ -1074,8 +1084,8 @@ inline int lanes_volumes(const DevLayout &L) { return L.level == 5 ? L.nspec : L
 // wavefront (e % VL) / (VL / W).  The precipitation-formation entries are at
 // most 8 neighbours: they start at their partial's place in a quad of the
 // tree, and the parity of that quad says how the (up to three) quads add up.
-int sweep_program(const DevLayout &L, bool hyd, uint32_t *prog) {
-  const int NV = lanes_volumes(L), W = !hyd ? kWavesA : NV > 2 ? kWaves4 : kWaves2, VL = !hyd ? kPartA : NV > 2 ? kPart4 : kPart2, A = VL / W;
+int sweep_program(const DevLayout &L, int kt, bool hyd, uint32_t *prog) {
+  const int NV = lanes_volumes(L), W = !hyd ? kWavesA : NV > 2 ? kWaves4 : kWaves2, VL = !hyd ? kPartA : NV == 2 ? kPart2 : L.level == 5 && kt == 8 ? kPart5d : kPart4, A = VL / W;
   const int kEnt = prog_entries(W);
   const int i0 = hyd ? 0 : L.it_aero0, nt = hyd ? L.ntarget : L.it_aero1 - L.it_aero0;
   const uint32_t zero = hyd ? L.npair : L.npair_aa;
@@ -1110,7 +1120,7 @@ int sweep_program(const DevLayout &L, bool hyd, uint32_t *prog) {
       if (at >= kEnt) return -1;
       out[((size_t)it * W + v) * kProg + at] = pair << 15 | j << 9 | role;
       if (!(role & SR_PF)) continue;
-      if (pf0 < 0) pf0 = VL == 16 ? e - e % 4 : e;
+      if (pf0 < 0) pf0 = VL >= 16 ? e - e % 4 : e;
       if (e - pf0 >= prog_pf(VL)) return -1;
       for (int u = 0; u < W; ++u) {
         uint32_t *p = out + ((size_t)it * W + u) * kProg;
@@ -1148,15 +1158,15 @@ bool lanes_fit(const DevLayout &L, int kt, int64_t ncells) {
   const int VL = NV == 2 ? kPart2 : kPart4, bins = VL * (NV == 2 ? kBins2 : kBins4);
   const bool fits = L.nt - L.in2a <= bins && L.nb[0] - L.in2a <= kPartA * kBinsA && pairs_lds(L.nt, kt, 32) <= kMaxLds &&
                     pairs_lds(L.nb[0], kt, kL) <= kMaxLds && sweep_lds(L.nt, NV, NV == 2 ? kWaves2 : kWaves4, L.ncc, L.nb[3]) <= kMaxLds;
-  return fits && L.lscoag && !L.lsdistupdate && !L.autoconv2 && !L.lsactiv && lanes_program(L, nullptr) > 0;
+  return fits && L.lscoag && !L.lsdistupdate && !L.autoconv2 && !L.lsactiv && lanes_program(L, kt, nullptr) > 0;
 }
 
 // The sweep programs with and then without hydrometeors; returns their words,
 // -1 where the layout does not fit.
-int lanes_program(const DevLayout &L, uint32_t *prog) {
-  const int n = sweep_program(L, true, prog);
+int lanes_program(const DevLayout &L, int kt, uint32_t *prog) {
+  const int n = sweep_program(L, kt, true, prog);
   if (n < 0) return -1;
-  const int m = sweep_program(L, false, prog ? prog + n : nullptr);
+  const int m = sweep_program(L, kt, false, prog ? prog + n : nullptr);
   return m < 0 ? -1 : n + m;
 }
 
@@ -1174,7 +1184,7 @@ size_t lanes_work(const DevLayout &L, int kt, int64_t ncells, LanesArgs &w) {
   w.o_dwa = take((size_t)sh * L.nb[0] * 8);
   w.o_dwaa = take((size_t)sa * L.nb[0] * 8);
   w.o_rows = take((size_t)L.nt * (1 + lanes_volumes(L)) * sizeof(LaneRow));
-  w.o_prog = take((size_t)lanes_program(L, nullptr) * sizeof(uint32_t));
+  w.o_prog = take((size_t)lanes_program(L, kt, nullptr) * sizeof(uint32_t));
   return o;
 }
 
@@ -1191,7 +1201,7 @@ int launch_lanes(const DevLayout &L, int precision, bool hyd, const DevLayout *d
   LanesArgs w = w0;
   const int NV = lanes_volumes(L);
   if (!hyd) {
-    w.prog += sweep_program(L, true, nullptr);
+    w.prog += sweep_program(L, precision == SALSA_FP64 ? 8 : 4, true, nullptr);
     w.K = w.Ka;
     w.dwa = w.dwaa;
   }
@@ -1202,8 +1212,8 @@ int launch_lanes(const DevLayout &L, int precision, bool hyd, const DevLayout *d
   if (precision == SALSA_FP64) {
     if (NV == 2) SALSA_LANES(double, 2, false, 8, kWaves2, kPart2, kBins2);
     if (NV == 3 && !l5) SALSA_LANES(double, 3, false, 8, kWaves4, kPart4, kBins4);
-    if (NV == 3) SALSA_LANES(double, 3, true, 8, kWaves4, kPart4, kBins4);
-    SALSA_LANES(double, 4, true, 8, kWaves4, kPart4, kBins4);
+    if (NV == 3) SALSA_LANES(double, 3, true, 8, kWaves4, kPart5d, kBins5d);
+    SALSA_LANES(double, 4, true, 8, kWaves4, kPart5d, kBins5d);
   }
   if (NV == 2) SALSA_LANES(float, 2, false, 4, kWaves2, kPart2, kBins2);
   if (NV == 3 && !l5) SALSA_LANES(float, 3, false, 4, kWaves4, kPart4, kBins4);
