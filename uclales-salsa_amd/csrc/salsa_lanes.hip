@@ -515,6 +515,10 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
     if (!__any(act)) continue;                          // the same in every wavefront of the block
     const bool ice = HYD && L5 && (fl & TF_ICE);
     const double rft = ice ? sRF[(t - Ioff) * kL + lane] : 0.;
+    // the last wavefront forms the target's new rime fraction from its old water
+    // and rime, which their owners overwrite beyond the next barrier
+    const bool rimer = ice && wv == W - 1;
+    const double old_w = rimer ? SC(t, 1 + iwa) : 0., old_r = rimer ? SC(t, 1 + irim) : 0.;
     const int nu = ice ? NV : nwet;                     // components that the target updates
     // a component's owner also moves what coalesces into precipitation
     KT kf[NF];
@@ -604,12 +608,12 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
     // another bin meets no other wavefront
     const double kself = (double)k.self;
     if constexpr (HYD && L5) {
-      if (ice && wv == W - 1) {                         // the target's rime fraction after its update
+      if (rimer) {                                      // the target's rime fraction after its update
         const double *pp = sP + lane;
         const double sk = tree_sum<W>(pp, NP * kL), ss = (emax - rft * (emax - emin)) * 0.5 * kself * Nt;
         const double nn = Nt * rcp_nr(1. + dt * (sk + ss)), rd = rcp_nr(1. + dt * sk);
-        const double vw = (SC(t, 1 + iwa) + dt * tree_sum<W>(pp + (1 + iwa) * kL, NP * kL) * Nt) * rd;
-        const double vr = (SC(t, 1 + irim) + dt * tree_sum<W>(pp + (1 + irim) * kL, NP * kL) * Nt) * rd;
+        const double vw = (old_w + dt * tree_sum<W>(pp + (1 + iwa) * kL, NP * kL) * Nt) * rd;
+        const double vr = (old_r + dt * tree_sum<W>(pp + (1 + irim) * kL, NP * kL) * Nt) * rd;
         if (act) sRF[(t - Ioff) * kL + lane] = rime(nn, vw, vr);
       }
     }
