@@ -50,3 +50,49 @@ def test_one_lane_step_with_ice_repeats_its_bits(capi, species, prec):
         for a, b in zip(out, want):
             assert torch.equal(a, b)
     ctx.close()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("level", [4, 5])
+def test_nan_and_negative_masses_of_inactive_bins(capi, level, prec):
+    """Masses of a hydrometeor bin below its number limit that are NaN or negative
+    are empty after a step and add nothing to a cell's water: the one-lane step
+    agrees with the general kernel (at 16 and 32 lanes), which clamps them first.
+
+    The bar is that of the comparison of the two paths elsewhere: 2^-53 on some
+    30 terms, grown by 1.1^50 = 117 in the substeps times a conditioning of 1e3,
+    1e-9 of an element; 1e-12 of a row's rms for what a process empties; ten
+    times what the general kernel moves between two shapes."""
+    print("case NaN in inactive bins, level %d prec %d" % (level, prec), flush=True)
+    desc, f = fields(capi, ("SO4",), level, (41, 20, 20), rh_range=(0.99, 1.01))
+    g, ncat = f.grid, 4 if level == 5 else 3
+    idx = g.interior_index()
+    n, m = [x.copy() for x in f.n[:ncat]], [x.copy() for x in f.m[:ncat]]
+    for c in range(1, ncat):                                # (level 5 has ice in every cell)
+        n[c][:, idx[::2]] = 0.
+        m[c][:, idx[::2]] = 0.
+    has = np.zeros(len(idx), bool)
+    for c in range(1, ncat):
+        has |= (n[c][:, idx] > 0.).any(axis=0)
+    off = idx[~has]
+    assert len(off) > 1000
+    water = desc.iwa * np.array([desc.nbins, desc.ncld, desc.nprc, desc.nice])
+    for c in range(1, ncat):
+        m[c][water[c], off[c::4]] = np.nan
+        m[c][water[c] + 1, off[c::3]] = -1.e-4
+        m[c][water[c] + 2, off[c::5]] = 1.e-9
+    res = []
+    for shape in (0, 16, 32):
+        ctx = capi.Context(desc, capi.params(level=level, precision=prec), g.nzp, g.nxp, g.nyp)
+        for k in range(3 if shape else 0):
+            ctx.set_shape(k, shape)
+        a, b = [x.copy() for x in n], [x.copy() for x in m]
+        fd = {k: np.array(getattr(f, k)) for k in ("press", "temp", "rsl", "rsi", "dn", "rv")}
+        ctx.step_host(fd, a, b, flags=capi.STEP_INPLACE)        # raises where a cell is not finite
+        res.append(([x[:, idx] for x in a + b + [fd["rv"][None]]], ctx.cell_flags()))
+        ctx.close()
+    assert np.array_equal(res[0][1], res[1][1])
+    for x, y, y2 in zip(res[0][0], res[1][0], res[2][0]):
+        rms = np.sqrt(np.mean(y * y, axis=1, keepdims=True))
+        bad = ~(np.abs(x - y) <= 1e-9 * np.abs(y) + 1e-12 * rms + 10. * np.abs(y - y2))
+        assert not bad.any(), (np.argwhere(bad)[:3], x[bad][:3], y[bad][:3], y2[bad][:3])

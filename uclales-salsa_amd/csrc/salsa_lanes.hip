@@ -447,7 +447,7 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
       for (int u = 0; u < RB; ++u)
         if (r0 + u < nall) {
           some |= live && !(v[u] == 0.);
-          if (w.rows[r0 + u].kind & LR_WATER) wat += v[u] * dn / kMwa;
+          if (w.rows[r0 + u].kind & LR_WATER) wat += fmax(0., v[u] * dn) / kMwa;   // (as the clamp leaves it)
         }
     }
     some = __any(some);
