@@ -1236,7 +1236,10 @@ extern "C" int salsa_sedim_device(salsa_ctx *c, double dtlt, const double *dzt, 
   a.nzp = c->nzp; a.nxp = c->nxp; a.nyp = c->nyp; a.level = P.level; a.n3 = c->n3; a.dtlt = dtlt;
   a.nb[0] = d.nbins; a.nb[1] = d.ncld; a.nb[2] = d.nprc; a.nb[3] = l5 ? d.nice : 0;
   a.ns = d.iwa + 1; a.ns_ice = d.iwa + 2; a.iwa = d.iwa; a.irim = d.irim;
-  for (int s = 0; s < SALSA_MAXSPEC; ++s) { a.rrholiq[s] = 1. / d.rholiq[s]; a.rrhoice[s] = 1. / d.rhoice[s]; }
+  for (int s = 0; s < SALSA_MAXSPEC; ++s) {
+    a.rholiq[s] = d.rholiq[s]; a.rhoice[s] = d.rhoice[s];
+    a.rrholiq[s] = 1. / d.rholiq[s]; a.rrhoice[s] = 1. / d.rhoice[s];
+  }
   a.ice_alpha = P.ice_alpha; a.ice_beta = P.ice_beta; a.ice_gamma = P.ice_gamma; a.ice_sigma = P.ice_sigma;
   for (int k = 0; k < c->nzp; ++k) {
     if (!(dzt[k] > 0.)) { set_error("dzt must be positive"); return SALSA_ERR_ARG; }

@@ -280,7 +280,7 @@ struct SedArgs {
   double dtlt;
   int32_t nb[4];                      // aerosol, cloud, precipitation, ice bins
   int32_t ns, ns_ice, iwa, irim;      // mass rows per bin (liquid: wet species; ice: + rime); water, rime
-  double rrholiq[kMaxSpec], rrhoice[kMaxSpec];        // 1 / density
+  double rholiq[kMaxSpec], rhoice[kMaxSpec], rrholiq[kMaxSpec], rrhoice[kMaxSpec];   // densities and 1 / density
   double ice_alpha, ice_beta, ice_gamma, ice_sigma;   // mo_ice_shape.f90:25-30
   double dzt[256];                    // inverse level thicknesses (nzp <= 256)
   const double *tk, *th, *adn, *ustar;

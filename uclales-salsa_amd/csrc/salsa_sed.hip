@@ -45,33 +45,42 @@ constexpr int kSedSpec = 3;                   // mass rows of a liquid bin that 
 constexpr double kPiFull = 3.14159265358979323846, kKb = 1.3807e-23, kG = 9.81, kCp = 1005., kAlvl = 2.5e6;
 constexpr double kLn10 = 2.302585092994045684;
 
-// Air at one level: viscosity, mean free path, and the quotients that every
-// bin's fall speed takes from them (divisions are the larger part of it).
-struct Air { double avis, lambda, il, iv, nu; };   // il 1 / (2 lambda), iv 1 / avis, nu avis / density
+// x / d from the reciprocal r of d (to a few units in its last place): the
+// residual of the product, formed exactly, corrects it to the correctly rounded
+// quotient.  A divisor that many quotients share costs each of them three
+// operations instead of a division's eleven.
+__device__ __forceinline__ double sd_quot(double x, double d, double r) {
+  const double q = x * r;
+  return __builtin_fma(__builtin_fma(-q, d, x), r, q);
+}
+
+// Air at one level: viscosity, twice the mean free path, their reciprocals (every
+// bin's fall speed divides by them), the viscosity over the density.
+struct Air { double avis, iv, l2, il, nu; };
 __device__ __forceinline__ Air sd_air(double tk, double adn) {
   Air a;
   const double tr = tk / 296.16;
   a.avis = 1.8325e-5 * (416.16 / (tk + 120.0)) * (tr * ::sqrt(tr));
   const double va = ::sqrt(8 * kKb * tk / (kPiFull * 4.8096e-26));
-  a.lambda = 2 * a.avis / (adn * va);
-  a.il = 0.5 / a.lambda;
+  a.l2 = 2. * (2 * a.avis / (adn * va));
+  a.il = 1. / a.l2;
   a.iv = 1. / a.avis;
   a.nu = a.avis / adn;
   return a;
 }
 
-// rdiam: 1 / diam
+// rdiam: 1 / diam, as sd_quot takes it
 __device__ __forceinline__ double sd_terminal_vel(double diam, double rdiam, double rhop, double rhoa, const Air &air,
                                                   double beta) {
-  if (diam <= 19e-6) return (diam * diam) * (rhop - rhoa) * kGrav * beta * air.iv * (1. / 18.);
+  if (diam <= 19e-6) return sd_quot((diam * diam) * (rhop - rhoa) * kGrav * beta, 18. * air.avis, air.iv * (1. / 18.));
   if (diam > 19e-6 && diam < 1.07e-3) {
-    const double NDa = 4. / 3. * (diam * diam * diam) * kGrav * (rhop - rhoa) * rhoa * (air.iv * air.iv);
+    const double NDa = sd_quot(4. / 3. * (diam * diam * diam) * kGrav * (rhop - rhoa) * rhoa, air.avis * air.avis, air.iv * air.iv);
     const double X = ::log(NDa);
     const double X2 = X * X, X3 = X2 * X, X4 = X2 * X2, X5 = X4 * X, X6 = X3 * X3;
     const double Y = -0.318657e1 + 0.992696 * X - 0.153193e-2 * X2 - 0.987059e-3 * X3 - 0.578878e-3 * X4 +
                      0.855176e-4 * X5 - 0.327815e-5 * X6;
     const double Re2 = beta * ::exp(Y);
-    return air.nu * rdiam * Re2;
+    return sd_quot(air.nu, diam, rdiam) * Re2;
   }
   // Np**(1/6) through log(Np) / 6: X3 = log(Bo) + log(Np) / 6 and
   // Re3 = exp(log(Np) / 6 + Y3), within a few 1e-16 of the powers
@@ -84,17 +93,21 @@ __device__ __forceinline__ double sd_terminal_vel(double diam, double rdiam, dou
   const double Y3 = -0.500015e1 + 0.523778e1 * X3 - 0.204914e1 * Z2 + 0.475294 * Z3 - 0.542819e-1 * Z4 +
                     0.238449e-2 * Z5;
   const double Re3 = ::exp(L6 + Y3);
-  return fmin(air.nu * rdiam * Re3, 9.2);
+  return fmin(sd_quot(air.nu, diam, rdiam) * Re3, 9.2);
 }
 
 // the bin's wet diameter, density, slip correction and fall speed from the
-// bin's number zpn >= 1e-15, volume v = sum m_s / rho_s and mass ms = sum m_s;
-// the density ms / zpn over the volume kPi6 dwet**3 = v / zpn of a particle
+// bin's number zpn >= 1e-15, volume v = sum m_s / rho_s and mass ms = sum m_s.
+// (The density is formed with the diameter although it is ms / v: in the product
+// of the diameter's cube and the density the rounding of the cube root cancels.)
 __device__ __forceinline__ double sd_vc_sums(double zpn, double v, double ms, double adn, const Air &air,
                                              double *dwet_out, double *gg_out) {
-  const double dwet = cbrt_fast(div_nr(v, zpn) * (1. / kPi6)), rdwet = rcp_nr(dwet);
-  const double zdn = div_nr(ms, v);
-  const double GG = 1. + 2. * air.lambda * rdwet * (1.249 + 0.42 * ::exp(-0.87 * (dwet * air.il)));
+  const double rn = rcp_nr(zpn);
+  const double dwet = cbrt_fast(sd_quot(sd_quot(v, zpn, rn), kPi6, 1. / kPi6)), rdwet = rcp_nr(dwet);
+  const double vp = kPi6 * (dwet * dwet * dwet);
+  const double zdn = sd_quot(sd_quot(ms, zpn, rn), vp, rcp_nr(vp));
+  const double Kn = dwet == 0. ? HUGE_VAL : sd_quot(air.l2, dwet, rdwet);
+  const double GG = 1. + Kn * (1.249 + 0.42 * ::exp(sd_quot(-0.87 * dwet, air.l2, air.il)));
   if (dwet_out) *dwet_out = dwet;
   if (gg_out) *gg_out = GG;
   return sd_terminal_vel(dwet, rdwet, zdn, adn, air, GG);
@@ -151,7 +164,7 @@ __global__ void __launch_bounds__(kSedMaxZ, MS <= 3 ? 3 : 1) k_sed_slow(SedArgs 
   double *__restrict__ Nt = a.n_t[cat];
   double *__restrict__ Mt = a.m_t[cat];
   double ad = 1., dz = 0., cap = 0., tkx = 0., ust = 0.;
-  Air ar{0., 0.};
+  Air ar{};
   if (src) {
     ad = a.adn[x];
     tkx = a.tk[x];
@@ -196,7 +209,7 @@ __global__ void __launch_bounds__(kSedMaxZ, MS <= 3 ? 3 : 1) k_sed_slow(SedArgs 
       double v = 0., ms = 0.;
 #pragma unroll
       for (int s = 0; s < MS; ++s)
-        if (s < ns) v = v + m[s] * a.rrholiq[s];
+        if (s < ns) v = v + sd_quot(m[s], a.rholiq[s], a.rrholiq[s]);
 #pragma unroll
       for (int s = 0; s < MS; ++s)
         if (s < ns) ms = ms + m[s];
@@ -289,45 +302,50 @@ size_t sed_slow_lds_bytes(int Z, int nb, int MS) {
 // Dgr = (alpha / (pi6 rho_b))**(1/(3-beta)), Dcr = Dgr h**(1/(3-beta))),
 // the Best number X = 2 vb (rhop-rhoa) g / (gamma rhoa visc**2) D**(2-sigma)
 // and the speed Are / X**bre * visc**(1-2 bre) * (2 alpha g / (rhoa gamma))**bre
-// * D**bv as one exponential: four logarithms (five for partly rimed ice) and
-// two exponentials per bin instead of eight powers, within a few 1e-14 of the
-// power form.  numc: the number, v, ms: volume sum m / rho and mass sum m of
-// the bin; lvisc, lrhoa: logarithms of the level's viscosity and density; c:
-// those of the constants.
-struct IceLogC { double lmth, lia, lpi6ic, lga, lpi4, l2g, inv, rib; };   // inv 1 / (3 - beta), rib 1 / beta
+// * D**bv as one exponential: five logarithms and two exponentials per bin
+// instead of eight powers, within a few 1e-14 of the power form.  The constants
+// and the level's viscosity and density go into the arguments of the logarithms
+// of X and of the factor, not in as logarithms of their own, whose roundings are
+// larger than the result.  numc: the number, v, ms: volume sum m / rho and mass
+// sum m of the bin; visc, lvisc, rv2: the level's viscosity, its logarithm and
+// 1 / visc**2; rrhoa: 1 / rhoa; c: of the constants.
+struct IceLogC { double lmth, lia, lpi6ic, rga, inv, rib; };   // rga 1 / gamma, inv 1 / (3 - beta), rib 1 / beta
 __device__ __forceinline__ double ice_vc_log(const SedArgs &a, const IceLogC &c, double v, double ms, double rhoa,
-                                             double lvisc, double lrhoa, double mpri, double mrim, double numc) {
-  double lal = c.lpi6ic, be = 3., lga = c.lpi4, si = 2.;
+                                             double visc, double lvisc, double rv2, double rrhoa, double mpri, double mrim,
+                                             double numc) {
+  double al = kPi6 * kRhoic, be = 3., ga = kPi / 4., rga = 4. / kPi, si = 2.;
   double Ld = -20.72326583694641;               // log(1e-9): getDiameter's value below the number limit
   const double rn = rcp_nr(numc);
   if (!(numc < 1.e-6)) {
-    const double mt = mpri + mrim, mtot = mt * rn;
-    const double fr = fmax(fmin(div_nr(mrim, mt), 0.9999), 0.0001);
+    const double mtot = sd_quot(mpri + mrim, numc, rn), mt = mtot * numc;
+    const double fr = fmax(fmin(sd_quot(mrim, mt, rcp_nr(mt)), 0.9999), 0.0001);
     const double rho_b = fr * kRhori + (1. - fr) * kRhoic;
     const double Lm = ::log(mtot), Lrb = ::log(kPi6 * rho_b);
     const double lmgr = Lrb + 3. * ((c.lia - Lrb) * c.inv);
-    const double Lh = -::log(1. - fr);
+    const double h = sd_quot(1., 1. - fr, rcp_nr(1. - fr)), Lh = ::log(h);
     const double lmcr = lmgr + 3. * (Lh * c.inv);
     if (Lm >= c.lmth && Lm < lmgr) {
-      lal = c.lia; be = a.ice_beta; lga = c.lga; si = a.ice_sigma;
+      al = a.ice_alpha; be = a.ice_beta; ga = a.ice_gamma; rga = c.rga; si = a.ice_sigma;
     } else if (Lm > lmcr) {
-      lal = c.lia + Lh; be = a.ice_beta; si = a.ice_sigma * (1. - fr) + 2. * fr;
-      lga = ::log(a.ice_gamma * (1. - fr) + kPi / 4. * fr);
+      al = a.ice_alpha * h; be = a.ice_beta; si = a.ice_sigma * (1. - fr) + 2. * fr;
+      ga = a.ice_gamma * (1. - fr) + kPi / 4. * fr;
+      rga = rcp_nr(ga);
     }
-    if (Lm < c.lmth) Ld = (Lm - c.lpi6ic) * (1. / 3.);
-    else if (Lm < lmgr) Ld = (Lm - c.lia) * c.rib;
-    else if (Lm < lmcr) Ld = (Lm - Lrb) * (1. / 3.);
-    else if (Lm >= lmcr) Ld = (Lm - Lh - c.lia) * c.rib;
+    if (Lm < c.lmth) Ld = sd_quot(Lm - c.lpi6ic, 3., 1. / 3.);
+    else if (Lm < lmgr) Ld = sd_quot(Lm - c.lia, a.ice_beta, c.rib);
+    else if (Lm < lmcr) Ld = sd_quot(Lm - Lrb, 3., 1. / 3.);
+    else if (Lm >= lmcr) Ld = sd_quot(Lm - Lh - c.lia, a.ice_beta, c.rib);
   }
   const double c1 = 0.0902, delta0 = 9.06;
-  const double lgr = lga + lrhoa;
-  const double LX = ::log(2. * kGrav * (v * rn) * (div_nr(ms, v) - rhoa)) - lgr - 2. * lvisc + (2. - si) * Ld;
-  const double sX = ::exp(0.5 * LX);
+  const double dsph = cbrt_fast(sd_quot(sd_quot(v, numc, rn), kPi6, 1. / kPi6)), vb = kPi6 * cubed(dsph);
+  const double zdn = sd_quot(sd_quot(ms, numc, rn), vb, rcp_nr(vb)), rgr = rga * rrhoa;
+  const double LX = ::log(sd_quot(2. * vb * (zdn - rhoa) * kGrav, ga * rhoa * visc * visc, rgr * rv2)) + (2. - si) * Ld;
+  const double sX = ::sqrt(::exp(LX));
   const double k1213 = ::sqrt(1. + c1 * sX), k1 = k1213 - 1.;
-  const double bre = div_nr(0.5 * c1 * sX, k1 * k1213);
+  const double bre = 0.5 * c1 * sX / k1 / k1213;
   const double bv = bre * (be - si + 2.) - 1.;
-  return 0.25 * delta0 * delta0 * k1 * k1 *
-         ::exp(-bre * LX + (1. - 2. * bre) * lvisc + bre * (c.l2g + lal - lgr) + bv * Ld);
+  const double Lc = ::log(sd_quot(2. * al * kGrav, rhoa * ga, rgr));
+  return 0.25 * delta0 * delta0 * k1 * k1 * ::exp(-bre * LX + (1. - 2. * bre) * lvisc + bre * Lc + bv * Ld);
 }
 
 // LDS of one column (Z = blockDim.x levels), carved from the dynamic buffer
@@ -344,12 +362,15 @@ __host__ __device__ inline size_t sed_prc_lds_bytes(int Z, int nb, int ns, int M
 // Bound by the fall speed's FP64 arithmetic and, at level 4, HBM.  One barrier
 // per bin: a source publishes its content and the two shares, and every level
 // scans the sources above it once for all quantities.  With a barrier and a
-// scan per bin and moved quantity (35 and 21 of them) and true divisions the
-// ice launch took 925 us at 128 x 128 x 100 cells and the precipitation launch
-// 141 us at 64 x 64 x 120; now 590 and 94 us. (Three wavefronts per SIMD without
-// the few spills of four: the same times; two: a fifth longer.)
+// scan per bin and moved quantity (35 and 21 of them) the ice launch took 929 us
+// at 128 x 128 x 100 cells and the precipitation launch 127 us at 64 x 64 x 120;
+// now 707 and 108 us, with the fall speeds' bits as they were.  (Reciprocals
+// without sd_quot's correction: 617 and 98 us, but fall speeds further from the
+// exact value, 5.3 against 4.6 units of 2^-53 rms.  Four wavefronts per SIMD,
+// with 14 to 34 spills, 698 and 124 us before the ice speed took its
+// diameter again, three 652 and 108 us.)
 template <int MS, bool ICE>
-__global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
+__global__ void __launch_bounds__(kSedMaxZ, 3) k_sed_prc(SedArgs a) {
   extern __shared__ double smem[];
   constexpr int cat = ICE ? 3 : 2;
   constexpr double alv = ICE ? kAls : kAlvl;
@@ -386,17 +407,15 @@ __global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
     }
   };
   load(0, qv, tv);
-  Air air = {0., 0., 0., 0., 0.};
-  double rr = 0., sw = 0., sr = 0., ad = 0., lvisc = 0., lrhoa = 0.;
-  IceLogC ilc{0., 0., 0., 0., 0., 0., 0., 0.};          // ice: log Mth (pristine threshold), log alpha, log(pi6 rhoic), ..
+  Air air{};
+  double rr = 0., sw = 0., sr = 0., ad = 0., lvisc = 0., rv2 = 0., rrhoa = 0.;
+  IceLogC ilc{};                                        // ice: log Mth (pristine threshold), log alpha, log(pi6 rhoic), ..
   if (ICE) {
     const double dth = ::pow(kPi6 * kRhoic / a.ice_alpha, 1. / (a.ice_beta - 3.));
     ilc.lmth = ::log(kRhoic * kPi6 * cubed(dth));
     ilc.lia = ::log(a.ice_alpha);
     ilc.lpi6ic = ::log(kPi6 * kRhoic);
-    ilc.lga = ::log(a.ice_gamma);
-    ilc.lpi4 = ::log(kPi / 4.);
-    ilc.l2g = ::log(2. * kGrav);
+    ilc.rga = 1. / a.ice_gamma;
     ilc.inv = 1. / (3. - a.ice_beta);
     ilc.rib = 1. / a.ice_beta;
   }
@@ -409,7 +428,8 @@ __global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
     air = sd_air(a.tk[x], ad);
     if (ICE) {
       lvisc = ::log(air.avis);
-      lrhoa = ::log(ad);
+      rv2 = air.iv * air.iv;
+      rrhoa = 1. / ad;
     }
     rr = rate[x];
   }
@@ -428,7 +448,7 @@ __global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
 #pragma unroll
       for (int s = 0; s < MS; ++s)
         if (s < ns) {
-          v = v + qv[1 + s] * (ICE ? a.rrhoice : a.rrholiq)[s];
+          v = v + sd_quot(qv[1 + s], (ICE ? a.rhoice : a.rholiq)[s], (ICE ? a.rrhoice : a.rrholiq)[s]);
           ms = ms + qv[1 + s];
         }
 #pragma unroll
@@ -445,7 +465,7 @@ __global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
           if (s < ns - 1) mpri = mpri + qv[1 + s];
           if (s == ns - 1) mrim = qv[1 + s];
         }
-        vc = ice_vc_log(a, ilc, v, ms, ad, lvisc, lrhoa, mpri, mrim, zpn);
+        vc = ice_vc_log(a, ilc, v, ms, ad, air.avis, lvisc, rv2, rrhoa, mpri, mrim, zpn);
       } else {
         vc = sd_vc_sums(zpn, v, ms, ad, air, nullptr, nullptr);
       }
@@ -467,7 +487,8 @@ __global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
       const double pre = fdos * Sdz[kf];
       two = !(pre > 0.5);
       // the shares (:1229-1246), thinner or thicker levels included
-      f1 = (two ? pre : 1.) * Sdz[kf - 1] * Srdz[two ? kf : k];
+      const int kb = two ? kf : k;
+      f1 = sd_quot((two ? pre : 1.) * Sdz[kf - 1], Sdz[kb], Srdz[kb]);
       f0 = two ? 1. - pre : 0.;
       d = k - kf;                               // >= -1
       Sf1[pb * Z + k] = f1;
@@ -511,7 +532,7 @@ __global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
       for (int u = 0; u <= MS; ++u) {
         if (u > ns) break;
         const int64_t r = u == 0 ? (int64_t)b * n3 : ((int64_t)(u - 1) * nb + b) * n3;
-        (u == 0 ? Nt : Mt)[r + x] = tv[u] + out[u] * rdt;
+        (u == 0 ? Nt : Mt)[r + x] = tv[u] + sd_quot(out[u], dtlt, rdt);
         if (u - 1 == iw) sw = sw + out[u];
         if (ICE && u - 1 == ir) sr = sr + out[u];
       }
@@ -536,7 +557,7 @@ __global__ void __launch_bounds__(kSedMaxZ, 4) k_sed_prc(SedArgs a) {
   }
   if (src) rate[x] = rr;
   // the water rows and, for ice, the rime rows
-  if (lev && k <= ktop) a.tlt[x] = a.tlt[x] - ((sw + sr) * rdt) * (alv / kCp) * a.th[x] / a.tk[x];
+  if (lev && k <= ktop) a.tlt[x] = a.tlt[x] - ((sw + sr) / dtlt) * (alv / kCp) * a.th[x] / a.tk[x];
   if (k == 0) {
     // SUM(remprc((ns-1)*nb:ns*nb)) (ice: (ns-2)*nb:ns*nb), 1-based, one entry
     // before the water rows as written (:1256-1260)
