@@ -96,3 +96,76 @@ def test_nan_and_negative_masses_of_inactive_bins(capi, level, prec):
         rms = np.sqrt(np.mean(y * y, axis=1, keepdims=True))
         bad = ~(np.abs(x - y) <= 1e-9 * np.abs(y) + 1e-12 * rms + 10. * np.abs(y - y2))
         assert not bad.any(), (np.argwhere(bad)[:3], x[bad][:3], y[bad][:3], y2[bad][:3])
+
+
+def test_only_steps_take_the_step_work_space(capi):
+    """A context that never steps with one lane per cell (sedimentation, a chosen
+    launch shape) holds no work space of that step: what creating and using it
+    takes is its cell records, lists and flags, and 32 MB for the runtime's own
+    granules.  A context's first step makes the space, another one reuses it."""
+    import torch
+    desc, f = fields(capi, ("SO4",), 4, (60, 48, 48))
+    g = f.grid
+    free = lambda: (torch.cuda.synchronize(), torch.cuda.mem_get_info()[0])[1]
+    T = lambda a: torch.from_numpy(np.array(a)).cuda()
+    fd = {k: T(getattr(f, k)) for k in ("press", "temp", "rsl", "rsi", "dn", "rv")}
+    n, m = [T(x) for x in f.n[:3]], [T(x) for x in f.m[:3]]
+    out = [torch.zeros_like(x) for x in n + m + [fd["rv"]]]
+    step = lambda c: c.step_device(fd, n, m, out[:3], out[3:6], out[6])
+    warm = capi.Context(desc, capi.params(level=4), g.nzp, g.nxp, g.nyp)     # code and queues are loaded by now
+    step(warm)
+    warm.sync()
+    warm.close()
+    rows = 3 * (desc.nbins + desc.ncld + desc.nprc)                          # number and two masses
+    records = 8 * g.ncells * (2 * rows + 7) + 16 * g.ncells
+    start = free()
+    ctx = capi.Context(desc, capi.params(level=4), g.nzp, g.nxp, g.nyp)
+    for k in range(3):
+        ctx.set_shape(k, 16)
+    step(ctx)
+    ctx.sync()
+    assert start - free() < records + (32 << 20)
+    ctx.close()
+    ctx = capi.Context(desc, capi.params(level=4), g.nzp, g.nxp, g.nyp)
+    assert start - free() < records + (32 << 20)
+    step(ctx)
+    ctx.sync()
+    after = free()
+    step(ctx)
+    ctx.sync()
+    assert free() >= after                                                   # (other objects may go meanwhile)
+    ctx.close()
+
+
+@pytest.mark.parametrize("level,grid", [(4, (40, 16, 25)), (5, (40, 11, 11))])
+def test_first_step_of_a_context_within_a_capture(capi, level, grid):
+    """The first step makes its work space also within a stream capture; replays,
+    with other work between them, give the bits of an eager step."""
+    import torch
+    print("case first step captured, level %d" % level, flush=True)
+    desc, f = fields(capi, ("SO4",), level, grid)
+    g, ncat = f.grid, 4 if level == 5 else 3
+    T = lambda a: torch.from_numpy(np.array(a)).cuda()
+    fd = {k: T(getattr(f, k)) for k in ("press", "temp", "rsl", "rsi", "dn", "rv")}
+    n, m = [T(x) for x in f.n[:ncat]], [T(x) for x in f.m[:ncat]]
+    out = [torch.zeros_like(x) for x in n + m + [fd["rv"]]]
+    step = lambda c: c.step_device(fd, n, m, out[:ncat], out[ncat:2 * ncat], out[-1])
+    ctx = capi.Context(desc, capi.params(level=level), g.nzp, g.nxp, g.nyp)
+    step(ctx)
+    ctx.sync()
+    ctx.close()
+    want = [x.clone() for x in out]
+    ctx = capi.Context(desc, capi.params(level=level), g.nzp, g.nxp, g.nyp)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=torch.cuda.ExternalStream(ctx.stream), capture_error_mode="thread_local"):
+        step(ctx)
+    for _ in range(3):
+        for x in out:
+            x.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, want):
+            assert torch.equal(a, b)
+    ctx.close()

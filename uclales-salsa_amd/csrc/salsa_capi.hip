@@ -88,10 +88,14 @@ struct salsa_ctx {
   int32_t *lists = nullptr;
   int32_t *cls_count = nullptr;       // device [3]
   int32_t *cls_count_h = nullptr;     // pinned host [3]
-  // one-lane-per-cell step: its work space (null where the layout or the
-  // options need the general kernel); shape_set: the caller chose the general
-  // kernel's lanes per cell
+  // one-lane-per-cell step: its sweep program (null where the layout or the
+  // options need the general kernel) and its work space, allocated by the first
+  // step that takes it (lanes_none: there was no memory for it, the general
+  // kernel runs instead); shape_set: the caller chose the general kernel's
+  // lanes per cell
+  uint32_t *lanes_prog = nullptr;
   char *lanes_buf = nullptr;
+  bool lanes_none = false;
   LanesArgs lw;
   hipStream_t side = nullptr;         // the cells without hydrometeors, beside those with (null: one after the other)
   hipEvent_t fork = nullptr, join = nullptr;
@@ -197,7 +201,7 @@ static void release(salsa_ctx *c) {
   (void)hipFree(c->adj_buf);
   (void)hipFree(c->les_list);
   (void)hipFree(c->act_state);
-  (void)hipFree(c->lanes_buf);
+  (void)hipFree(c->lanes_prog); (void)hipFree(c->lanes_buf);
   for (hipStream_t q : c->copy_stream)
     if (q) (void)hipStreamDestroy(q);
   if (c->side) (void)hipStreamDestroy(c->side);
@@ -295,39 +299,14 @@ extern "C" int salsa_ctx_create(const salsa_bin_desc *desc, const salsa_params *
   }
   const int kt = c->params.precision == SALSA_FP64 ? 8 : 4;
   if (c->params.lscoag_mode == 1 && lanes_fit(c->hostL, kt, c->ncells)) {
-    std::memset(&c->lw, 0, sizeof(c->lw));
-    const size_t need = lanes_work(c->hostL, kt, c->ncells, c->lw);
-    if (hipMalloc(&c->lanes_buf, need) != hipSuccess) {
-      set_error("step work allocation failed");
-      return fail(SALSA_ERR_NOMEM);
-    }
-    c->lw.counts = c->cls_count;
-    c->lw.lists = c->lists;
-    c->lw.ncells = c->ncells;
-    c->lw.K = c->lanes_buf;
-    c->lw.Ka = c->lanes_buf + c->lw.o_Ka;
-    c->lw.dwaa = reinterpret_cast<double *>(c->lanes_buf + c->lw.o_dwaa);
-    c->lw.pf = reinterpret_cast<uint8_t *>(c->lanes_buf + c->lw.o_pf);
-    c->lw.dwa = reinterpret_cast<double *>(c->lanes_buf + c->lw.o_dwa);
-    c->lw.rows = reinterpret_cast<LaneRow *>(c->lanes_buf + c->lw.o_rows);
-    c->lw.prog = reinterpret_cast<const uint32_t *>(c->lanes_buf + c->lw.o_prog);
-    // The cells with and without hydrometeors run side by side where neither
-    // list fills the chip for long.  Measured us, one after the other / side by
-    // side: level 4 mixed 15 360 cells 246 / 192, 40 960 269 / 213, 81 920
-    // 356 / 339, with drizzle 362 / 260, FP64 433 / 398, 176 715 797 / 767; the
-    // deck of 491 520 cells 1 317 / 1 335; level 5 with ice everywhere (an empty
-    // second list) 10 240 255 / 259.
-    if (c->hostL.level == 4 && c->ncells <= (1 << 18) &&
-        (hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
-         hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) != hipSuccess ||
-         hipEventCreateWithFlags(&c->join, hipEventDisableTiming) != hipSuccess)) {
-      set_error("hipStreamCreate failed");
-      return fail(SALSA_ERR_HIP);
-    }
     std::vector<uint32_t> prog((size_t)lanes_program(c->hostL, kt, nullptr));
     (void)lanes_program(c->hostL, kt, prog.data());
-    if (hipMemcpy(c->lanes_buf + c->lw.o_prog, prog.data(), prog.size() * sizeof(uint32_t), hipMemcpyHostToDevice) !=
-        hipSuccess) {
+    const size_t n = prog.size() * sizeof(uint32_t);
+    if (hipMalloc(&c->lanes_prog, n) != hipSuccess) {
+      set_error("device allocation failed");
+      return fail(SALSA_ERR_NOMEM);
+    }
+    if (hipMemcpy(c->lanes_prog, prog.data(), n, hipMemcpyHostToDevice) != hipSuccess) {
       set_error("copy of the sweep program failed");
       return fail(SALSA_ERR_HIP);
     }
@@ -502,11 +481,57 @@ static StepArgs class_args(salsa_ctx *c, const StepArgs &a, int k) {
   return b;
 }
 
+// The work space of the one-lane-per-cell step, by the first step that takes it
+// (up to 0.4 GB of the 26-bin layout in FP32, 0.7 GB in FP64: contexts that never
+// step this way do without), also one within a stream capture.  False where there
+// is no memory for it.
+static bool lanes_ready(salsa_ctx *c) {
+  if (c->lanes_buf || c->lanes_none) return c->lanes_buf;
+  // Allocations, a stream and events leave a capture as it is.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  LanesArgs &w = c->lw;
+  std::memset(&w, 0, sizeof(w));
+  const int kt = c->params.precision == SALSA_FP64 ? 8 : 4;
+  const size_t need = lanes_work(c->hostL, kt, c->ncells, w);
+  bool ok = hipMalloc(&c->lanes_buf, need) == hipSuccess;
+  // The cells with and without hydrometeors run side by side where neither
+  // list fills the chip for long.  Measured us, one after the other / side by
+  // side: level 4 mixed 15 360 cells 246 / 192, 40 960 269 / 213, 81 920
+  // 356 / 339, with drizzle 362 / 260, FP64 433 / 398, 176 715 797 / 767; the
+  // deck of 491 520 cells 1 317 / 1 335; level 5 with ice everywhere (an empty
+  // second list) 10 240 255 / 259.
+  if (ok && c->hostL.level == 4 && c->ncells <= (1 << 18))
+    ok = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) == hipSuccess &&
+         hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) == hipSuccess &&
+         hipEventCreateWithFlags(&c->join, hipEventDisableTiming) == hipSuccess;
+  if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (!ok) {
+    (void)hipGetLastError();                  // not an error of the step, which the general kernel takes
+    (void)hipFree(c->lanes_buf);
+    c->lanes_buf = nullptr;
+    c->lanes_none = true;
+    return false;
+  }
+  w.counts = c->cls_count;
+  w.lists = c->lists;
+  w.ncells = c->ncells;
+  w.K = c->lanes_buf;
+  w.Ka = c->lanes_buf + w.o_Ka;
+  w.dwaa = reinterpret_cast<double *>(c->lanes_buf + w.o_dwaa);
+  w.pf = reinterpret_cast<uint8_t *>(c->lanes_buf + w.o_pf);
+  w.dwa = reinterpret_cast<double *>(c->lanes_buf + w.o_dwa);
+  w.rows = reinterpret_cast<LaneRow *>(c->lanes_buf + w.o_rows);
+  w.prog = c->lanes_prog;
+  return true;
+}
+
 // The step with one lane per cell (salsa_lanes.hip): coagulation and
 // condensation without the optional processes, diagnostics and call forms
 // that only the general kernel has.
-static bool use_lanes(const salsa_ctx *c, const StepArgs &a, int32_t flags) {
-  return c->lanes_buf && !c->shape_set && !a.rates && !a.init && !a.kmode && !(flags & SALSA_STEP_NO_COMPACT);
+static bool use_lanes(salsa_ctx *c, const StepArgs &a, int32_t flags) {
+  return c->lanes_prog && !c->shape_set && !a.rates && !a.init && !a.kmode && !(flags & SALSA_STEP_NO_COMPACT) &&
+         lanes_ready(c);
 }
 
 static int enqueue_lanes(salsa_ctx *c, const StepArgs &a) {
@@ -594,7 +619,7 @@ extern "C" int salsa_ctx_timing(salsa_ctx *c, int32_t enable) {
   c->ev_cells.clear();
   c->ev_slot.clear();
   c->ev_counts = 0;
-  if (enable && c->lanes_buf && !c->ev_counts_h)
+  if (enable && c->lanes_prog && !c->ev_counts_h)
     HIPCHK(hipHostMalloc(&c->ev_counts_h, 3 * kTimedCounts * sizeof(int32_t)));
   c->timing = enable != 0;
   return SALSA_OK;

@@ -193,7 +193,7 @@ struct LanesArgs {
   double *dwa;                        // wet diameters of the aerosol bins before the step [block][nbins][64]
   void *Ka;                           // K and dwa of the cells without hydrometeors
   double *dwaa;
-  size_t o_Ka, o_pf, o_dwa, o_dwaa, o_rows, o_prog;   // byte offsets in the work space
+  size_t o_Ka, o_pf, o_dwa, o_dwaa, o_rows;   // byte offsets in the work space
 };
 
 // Arguments of the forward-mode derivative kernel: the trajectory starts from

@@ -1188,7 +1188,6 @@ size_t lanes_work(const DevLayout &L, int kt, int64_t ncells, LanesArgs &w) {
   w.o_dwa = take((size_t)sh * L.nb[0] * 8);
   w.o_dwaa = take((size_t)sa * L.nb[0] * 8);
   w.o_rows = take((size_t)L.nt * (1 + lanes_volumes(L)) * sizeof(LaneRow));
-  w.o_prog = take((size_t)lanes_program(L, kt, nullptr) * sizeof(uint32_t));
   return o;
 }
 
