@@ -169,3 +169,31 @@ def test_first_step_of_a_context_within_a_capture(capi, level, grid):
         for a, b in zip(out, want):
             assert torch.equal(a, b)
     ctx.close()
+
+
+def test_class_counts_of_many_timed_steps(capi):
+    """salsa_ctx_phase_time adds up every timed step's own class counts, also past
+    the 4 096 steps whose counts travel without a wait: steps without hydrometeors,
+    but for twenty on both sides of that number with them in known cells."""
+    import torch
+    desc, f = fields(capi, ("SO4",), 4, (40, 16, 24))
+    g = f.grid
+    idx = torch.from_numpy(g.interior_index()).cuda()
+    T = lambda a: torch.from_numpy(np.array(a)).cuda()
+    fd = {k: T(getattr(f, k)) for k in ("press", "temp", "rsl", "rsi", "dn", "rv")}
+    n, m = [T(x) for x in f.n[:3]], [T(x) for x in f.m[:3]]
+    out = [torch.zeros_like(x) for x in n + m + [fd["rv"]]]
+    dry = [n[0]] + [torch.zeros_like(x) for x in n[1:]]
+    nhyd = int(((n[1][:, idx] > 0.).any(0) | (n[2][:, idx] > 0.).any(0)).sum())
+    assert 0 < nhyd < g.ncells
+    ctx = capi.Context(desc, capi.params(level=4), g.nzp, g.nxp, g.nyp)
+    ctx.timing(True)
+    steps = 4096 + 40
+    for k in range(steps):
+        ctx.step_device(fd, n if 4090 <= k < 4110 else dry, m, out[:3], out[3:6], out[6], tstep=0.02)
+    ms, cells, nsteps = ctx.phase_time()
+    ctx.timing(False)
+    ctx.close()
+    assert nsteps == steps
+    assert cells[2] == 20 * nhyd
+    assert sum(cells) == steps * g.ncells

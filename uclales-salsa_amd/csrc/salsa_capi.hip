@@ -126,7 +126,7 @@ struct salsa_ctx {
   std::vector<hipEvent_t> ev;
   std::vector<int64_t> ev_cells;      // [3] per timed step, read on the host by the general path
   int32_t *ev_counts_h = nullptr;     // pinned host [kTimedCounts][3]: class counts of the others
-  std::vector<int> ev_slot;           // per timed step: its place in ev_counts_h, -1 where ev_cells has it
+  std::vector<int> ev_slot;           // per timed step: its place in ev_counts_h, or where ev_cells has it
   int ev_counts = 0;
   // this device's copy of the static work space of the allocation-free entry
   double *scratch = nullptr;
@@ -134,7 +134,8 @@ struct salsa_ctx {
   int32_t *fault_h = nullptr;         // pinned host [1]: the OR of the cell flags
 };
 constexpr int kEvPerStep = 10;
-constexpr int kTimedCounts = 4096;    // timed steps whose class counts need no wait
+constexpr int kTimedCounts = 4096;    // timed steps of the one-lane path between two waits for their class counts
+enum { kCountsHost = -1, kCountsKept = -2 };   // ev_slot of the general path, and of the one-lane path once waited for
 
 // ---------------------------------------------------------------------------
 // Work space of salsa_gradient_device_noalloc: per-cell J, per-cell dJ/dE and
@@ -560,8 +561,16 @@ static int enqueue_lanes(salsa_ctx *c, const StepArgs &a) {
   MARK();
   if (rc) { std::snprintf(g_err, sizeof(g_err), "step launch failed (%d)", rc); return SALSA_ERR_HIP; }
   if (c->timing) {
-    const int i = c->ev_counts < kTimedCounts ? c->ev_counts++ : kTimedCounts - 1;
-    if (i == kTimedCounts - 1) HIPCHK(hipStreamSynchronize(s));
+    if (c->ev_counts == kTimedCounts) {       // full: wait for the counts and keep them on the host
+      HIPCHK(hipStreamSynchronize(s));
+      for (size_t st = 0; st < c->ev_slot.size(); ++st) {
+        if (c->ev_slot[st] < 0) continue;
+        for (int k = 0; k < 3; ++k) c->ev_cells[3 * st + k] = c->ev_counts_h[3 * c->ev_slot[st] + k];
+        c->ev_slot[st] = kCountsKept;
+      }
+      c->ev_counts = 0;
+    }
+    const int i = c->ev_counts++;
     HIPCHK(hipMemcpyAsync(c->ev_counts_h + 3 * i, c->cls_count, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
     c->ev_slot.push_back(i);
     c->ev_cells.insert(c->ev_cells.end(), 3, 0);
@@ -606,7 +615,7 @@ static int enqueue_step(salsa_ctx *c, StepArgs a, int32_t flags) {
   MARK();
   if (c->timing) {
     c->ev_cells.insert(c->ev_cells.end(), cells, cells + 3);
-    c->ev_slot.push_back(-1);
+    c->ev_slot.push_back(kCountsHost);
   }
   return SALSA_OK;
 }
@@ -640,6 +649,7 @@ extern "C" int salsa_ctx_phase_time(salsa_ctx *c, double ms[5], int64_t cells[3]
   for (size_t st = 0; st < n; ++st) {
     if (el(st, 0, 1, ms[0])) return SALSA_ERR_HIP;                 // gather + classification
     const int slot = c->ev_slot[st];
+    const bool lanes = slot != kCountsHost;
     int64_t n[3];
     double t[3] = {0., 0., 0.};
     for (int k = 0; k < 3; ++k) {
@@ -647,7 +657,7 @@ extern "C" int salsa_ctx_phase_time(salsa_ctx *c, double ms[5], int64_t cells[3]
       cells[k] += n[k];
       if (el(st, 2 + 2 * k, 3 + 2 * k, t[k])) return SALSA_ERR_HIP;        // class k step kernel
     }
-    if (slot >= 0 && n[0] + n[1] > 0) {        // one launch of both: its time by their cells
+    if (lanes && n[0] + n[1] > 0) {            // one launch of both: its time by their cells
       const double both = t[0];
       t[0] = both * (double)n[0] / (double)(n[0] + n[1]);
       t[1] = both - t[0];
