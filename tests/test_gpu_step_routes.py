@@ -197,3 +197,39 @@ def test_class_counts_of_many_timed_steps(capi):
     assert nsteps == steps
     assert cells[2] == 20 * nhyd
     assert sum(cells) == steps * g.ncells
+
+
+@pytest.mark.parametrize("grid", [(40, 16, 24), (20, 8, 8)])
+def test_autotune_keeps_a_chosen_launch_by_class(capi, grid):
+    """salsa_set_launch_shape selects launches by cost class for every step of the
+    context; salsa_autotune changes the shapes, not that choice: the step gives the
+    bits of a context whose shapes were set to what the autotuner found.  Without a
+    chosen shape the route stays the context's own."""
+    import torch
+    desc, f = fields(capi, ("SO4",), 4, grid)
+    g = f.grid
+    T = lambda a: torch.from_numpy(np.array(a)).cuda()
+    fd = {k: T(getattr(f, k)) for k in ("press", "temp", "rsl", "rsi", "dn", "rv")}
+    n, m = [T(x) for x in f.n[:3]], [T(x) for x in f.m[:3]]
+
+    def step(shapes, tune):
+        ctx = capi.Context(desc, capi.params(level=4), g.nzp, g.nxp, g.nyp)
+        for k, s in enumerate(shapes):
+            ctx.set_shape(k, s)
+        if tune:
+            ctx.autotune(fd, n, m)
+        out = [torch.zeros_like(x) for x in n + m + [fd["rv"]]]
+        ctx.step_device(fd, n, m, out[:3], out[3:6], out[6])
+        ctx.sync()
+        found = [ctx.shape_of(k) for k in range(3)]
+        ctx.close()
+        return out, found
+
+    tuned, found = step((64, 64, 64), True)
+    by_class, _ = step(found, False)
+    for a, b in zip(tuned, by_class):
+        assert torch.equal(a, b)
+    own, _ = step((), False)
+    after, _ = step((), True)
+    for a, b in zip(own, after):
+        assert torch.equal(a, b)

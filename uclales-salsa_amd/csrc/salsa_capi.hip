@@ -1125,9 +1125,10 @@ extern "C" int salsa_autotune(salsa_ctx *c, const double *press, const double *t
   }
   StepArgs a = make_args(c, press, temp, rsl, rsi, dn, rv_p, rvt, n_p, nt, m_p, mt, nullptr, tstep, 0);
   a.kmode = 0;                                           // tuning neither reads nor writes the kernel store
+  const bool chosen = c->shape_set;
   c->shape_set = true;                                   // the shapes are the general kernel's
   int rc = enqueue_step(c, a, 0);                        // classification + warm-up
-  c->shape_set = false;
+  c->shape_set = chosen;                                 // a caller's choice of launches by class stays
   if (rc) { hipFree(scr); return rc; }
   hipStream_t s = c->stream;
   hipEvent_t e0, e1;
