@@ -10,6 +10,7 @@
 #include <atomic>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <thread>
 #include <mutex>
 #include <new>
@@ -300,14 +301,15 @@ extern "C" int salsa_ctx_create(const salsa_bin_desc *desc, const salsa_params *
   }
   const int kt = c->params.precision == SALSA_FP64 ? 8 : 4;
   if (c->params.lscoag_mode == 1 && lanes_fit(c->hostL, kt, c->ncells)) {
-    std::vector<uint32_t> prog((size_t)lanes_program(c->hostL, kt, nullptr));
-    (void)lanes_program(c->hostL, kt, prog.data());
-    const size_t n = prog.size() * sizeof(uint32_t);
+    const size_t words = (size_t)lanes_program(c->hostL, kt, nullptr), n = words * sizeof(uint32_t);
+    const std::unique_ptr<uint32_t[]> prog(new (std::nothrow) uint32_t[words]);
+    if (!prog) { set_error("out of host memory"); return fail(SALSA_ERR_NOMEM); }
+    (void)lanes_program(c->hostL, kt, prog.get());
     if (hipMalloc(&c->lanes_prog, n) != hipSuccess) {
       set_error("device allocation failed");
       return fail(SALSA_ERR_NOMEM);
     }
-    if (hipMemcpy(c->lanes_prog, prog.data(), n, hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMemcpy(c->lanes_prog, prog.get(), n, hipMemcpyHostToDevice) != hipSuccess) {
       set_error("copy of the sweep program failed");
       return fail(SALSA_ERR_HIP);
     }

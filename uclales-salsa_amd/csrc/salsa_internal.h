@@ -186,7 +186,8 @@ struct LanesArgs {
   int32_t g0;                         // first block of 64 slots of this chunk
   int32_t gn_hyd, gn_aero;            // blocks that the work space holds with and without hydrometeor pairs
   LaneRow *rows;                      // the call's field rows in state order
-  const uint32_t *prog;               // the sweep program
+  const uint32_t *prog;               // the sweep programs with and, from word prog_aero on, without hydrometeors
+  int32_t prog_aero;
   // per block of the chunk, 64 cells side by side:
   void *K;                            // kernels [block][pair][64], a row of zeros last
   uint8_t *pf;                        // COUNT(D_new > precpbins) per cloud-cloud pair [block][ncc][64]

@@ -38,7 +38,6 @@
 
 #include <cmath>
 #include <cstring>
-#include <vector>
 
 #include "salsa_internal.h"
 #include "salsa_physics.h"
@@ -1083,8 +1082,8 @@ constexpr int kPart5d = 32, kBins5d = 1;
 
 inline int lanes_volumes(const DevLayout &L) { return L.level == 5 ? L.nspec : L.nwet; }
 
-// The sweep program of the layout; returns its words, -1 where the layout does
-// not fit.  Entry e of a target is in partial e % VL, which belongs to
+// The sweep program of the layout (prog null: nothing written); returns its
+// words, -1 where the layout does not fit.  Entry e of a target is in partial e % VL, which belongs to
 // wavefront (e % VL) / (VL / W).  The precipitation-formation entries are at
 // most 8 neighbours: they start at their partial's place in a quad of the
 // tree, and the parity of that quad says how the (up to three) quads add up.
@@ -1094,8 +1093,7 @@ int sweep_program(const DevLayout &L, int kt, bool hyd, uint32_t *prog) {
   const int i0 = hyd ? 0 : L.it_aero0, nt = hyd ? L.ntarget : L.it_aero1 - L.it_aero0;
   const uint32_t zero = hyd ? L.npair : L.npair_aa;
   if (zero > 1023u || nt < 1) return -1;
-  std::vector<uint32_t> tmp(prog ? 0 : (size_t)nt * W * kProg);
-  uint32_t *out = prog ? prog : tmp.data();
+  auto set = [&](int it, int v, int q, uint32_t x) { if (prog) prog[((size_t)it * W + v) * kProg + q] = x; };
   for (int it = 0; it < nt; ++it) {
     const DevTarget &T = L.tgt[i0 + it];
     const bool self = T.flags & (TF_SELF_HALF | TF_SELF_HALF_EAGG | TF_PF_SELF | TF_PRECIP_SELFCOLL);
@@ -1103,15 +1101,14 @@ int sweep_program(const DevLayout &L, int kt, bool hyd, uint32_t *prog) {
     uint64_t bits;
     std::memcpy(&bits, &L.nlim[T.t], 8);
     for (int v = 0; v < W; ++v) {
-      uint32_t *p = out + ((size_t)it * W + v) * kProg;
-      for (int q = 0; q < kProg; ++q) p[q] = 0;
-      for (int q = 0; q < kEnt; ++q) p[q] = zero << 15 | (uint32_t)T.t << 9;
-      for (int q = 0; q < prog_pf(VL); ++q) p[kProgF + q] = zero | (uint32_t)T.t << 16;
-      p[kProgT] = (uint32_t)T.t | T.flags << 8;
-      p[kProgK] = pid >= 0 ? (uint32_t)pid : zero;
-      p[kProgN] = (uint32_t)bits;
-      p[kProgN + 1] = (uint32_t)(bits >> 32);
-      p[kProgS] = (T.flags & TF_PF_SELF) && pid >= 0 ? (uint32_t)(pid - L.pf0) : ~0u;
+      for (int q = 0; q < kProg; ++q) set(it, v, q, 0);
+      for (int q = 0; q < kEnt; ++q) set(it, v, q, zero << 15 | (uint32_t)T.t << 9);
+      for (int q = 0; q < prog_pf(VL); ++q) set(it, v, kProgF + q, zero | (uint32_t)T.t << 16);
+      set(it, v, kProgT, (uint32_t)T.t | T.flags << 8);
+      set(it, v, kProgK, pid >= 0 ? (uint32_t)pid : zero);
+      set(it, v, kProgN, (uint32_t)bits);
+      set(it, v, kProgN + 1, (uint32_t)(bits >> 32));
+      set(it, v, kProgS, (T.flags & TF_PF_SELF) && pid >= 0 ? (uint32_t)(pid - L.pf0) : ~0u);
     }
     int pf0 = -1;
     for (int e = 0; e < ne; ++e) {
@@ -1122,14 +1119,13 @@ int sweep_program(const DevLayout &L, int kt, bool hyd, uint32_t *prog) {
                             (r & R_FIX_OTH ? SR_FIX_OTH : 0);
       const int v = (e % VL) / A, at = (e / VL) * A + e % A;
       if (at >= kEnt) return -1;
-      out[((size_t)it * W + v) * kProg + at] = pair << 15 | j << 9 | role;
+      set(it, v, at, pair << 15 | j << 9 | role);
       if (!(role & SR_PF)) continue;
       if (pf0 < 0) pf0 = VL >= 16 ? e - e % 4 : e;
       if (e - pf0 >= prog_pf(VL)) return -1;
       for (int u = 0; u < W; ++u) {
-        uint32_t *p = out + ((size_t)it * W + u) * kProg;
-        p[kProgF + e - pf0] = pair | j << 16 | (r & R_PF_OWN ? 1u << 30 : 0u) | 1u << 31;
-        p[kProgQ] = (pf0 / 4) & 1;
+        set(it, u, kProgF + e - pf0, pair | j << 16 | (r & R_PF_OWN ? 1u << 30 : 0u) | 1u << 31);
+        set(it, u, kProgQ, (pf0 / 4) & 1);
       }
     }
   }
@@ -1174,7 +1170,8 @@ int lanes_program(const DevLayout &L, int kt, uint32_t *prog) {
   return m < 0 ? -1 : n + m;
 }
 
-// Work space of a context with ncells cells: byte offsets and the total.
+// Work space of a context with ncells cells: byte offsets and the total; where the
+// second sweep program begins.
 size_t lanes_work(const DevLayout &L, int kt, int64_t ncells, LanesArgs &w) {
   auto slots = [&](int most) { const int64_t n = (ncells + kL - 1) / kL * kL; return (int64_t)(n < most ? n : most); };
   const int64_t sh = slots(kSlotsHyd), sa = slots(kSlotsAero);
@@ -1188,6 +1185,7 @@ size_t lanes_work(const DevLayout &L, int kt, int64_t ncells, LanesArgs &w) {
   w.o_dwa = take((size_t)sh * L.nb[0] * 8);
   w.o_dwaa = take((size_t)sa * L.nb[0] * 8);
   w.o_rows = take((size_t)L.nt * (1 + lanes_volumes(L)) * sizeof(LaneRow));
+  w.prog_aero = sweep_program(L, kt, true, nullptr);
   return o;
 }
 
@@ -1204,7 +1202,7 @@ int launch_lanes(const DevLayout &L, int precision, bool hyd, const DevLayout *d
   LanesArgs w = w0;
   const int NV = lanes_volumes(L);
   if (!hyd) {
-    w.prog += sweep_program(L, precision == SALSA_FP64 ? 8 : 4, true, nullptr);
+    w.prog += w.prog_aero;
     w.K = w.Ka;
     w.dwa = w.dwaa;
   }
