@@ -233,3 +233,41 @@ def test_autotune_keeps_a_chosen_launch_by_class(capi, grid):
     after, _ = step((), True)
     for a, b in zip(own, after):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_one_lane_step_takes_the_layouts_ice_limit(capi, prec):
+    """The number below which an ice bin is empty is the layout's: with a lower one
+    than usual, and particles between the two, the one-lane step agrees with the
+    general kernel at two shapes (the bar of the comparison of the two paths above)."""
+    print("case ice limit of the layout, prec %d" % prec, flush=True)
+    desc, f = fields(capi, ("SO4",), 5, (41, 20, 12), t_range=(240., 270.))
+    g = f.grid
+    idx = g.interior_index()
+    ice0 = desc.nbins + desc.ncld + desc.nprc
+    for b in range(desc.nice):
+        desc.nlim[ice0 + b] = 1.e-12
+    n, m = [x.copy() for x in f.n], [x.copy() for x in f.m]
+    # every other bin with particles of its own mass, but some 1e-8 per kg of them, and mostly rimed: the others
+    # collect them at an efficiency that their rime fraction sets
+    water, rime = desc.iwa * desc.nice, desc.irim * desc.nice
+    m[3][rime:rime + desc.nice] = 0.1 * m[3][water:water + desc.nice]
+    for b in range(0, desc.nice, 2):
+        few = 1.e-8 / np.maximum(n[3][b], 1.e-8)
+        n[3][b] *= few
+        m[3][b::desc.nice] *= few
+        m[3][rime + b] = 3. * m[3][water + b]
+    res = []
+    for shape in (0, 16, 32):
+        ctx = capi.Context(desc, capi.params(level=5, precision=prec), g.nzp, g.nxp, g.nyp)
+        for k in range(3 if shape else 0):
+            ctx.set_shape(k, shape)
+        a, b = [x.copy() for x in n], [x.copy() for x in m]
+        fd = {k: np.array(getattr(f, k)) for k in ("press", "temp", "rsl", "rsi", "dn", "rv")}
+        ctx.step_host(fd, a, b, flags=capi.STEP_INPLACE)
+        res.append([x[:, idx] for x in a + b + [fd["rv"][None]]])
+        ctx.close()
+    for x, y, y2 in zip(*res):
+        rms = np.sqrt(np.mean(y * y, axis=1, keepdims=True))
+        bad = ~(np.abs(x - y) <= 1e-9 * np.abs(y) + 1e-12 * rms + 10. * np.abs(y - y2))
+        assert not bad.any(), (np.argwhere(bad)[:3], x[bad][:3], y[bad][:3], y2[bad][:3])

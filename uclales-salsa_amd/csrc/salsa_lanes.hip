@@ -464,11 +464,12 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
   const double emax = D.Eiagg_max, emin = D.Eiagg_min;
   // rime fraction of an ice bin (classSection.f90:202-224); kept per bin, as
   // a target's update is the only change to it
-  auto rime = [](double n, double wa, double ri) -> double {
-    return wa > 1.e-23 && ri > 1.e-23 && n > kPrlim ? ri * kRhori / (wa * kRhoic + ri * kRhori) : 0.;
+  auto rime = [](double n, double nlim, double wa, double ri) -> double {
+    return wa > 1.e-23 && ri > 1.e-23 && n > nlim ? ri * kRhori / (wa * kRhoic + ri * kRhori) : 0.;
   };
   if constexpr (HYD && L5) {
-    for (int q = wv; q < D.nb[3]; q += W) sRF[q * kL + lane] = rime(SC(Ioff + q, 0), SC(Ioff + q, 1 + iwa), SC(Ioff + q, 1 + irim));
+    for (int q = wv; q < D.nb[3]; q += W) sRF[q * kL + lane] =
+        rime(SC(Ioff + q, 0), D.nlim[Ioff + q], SC(Ioff + q, 1 + iwa), SC(Ioff + q, 1 + irim));
     __syncthreads();
   }
   // x / d for a constant d with reciprocal r: the correctly rounded quotient
@@ -613,7 +614,7 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
         const double nn = Nt * rcp_nr(1. + dt * (sk + ss)), rd = rcp_nr(1. + dt * sk);
         const double vw = (old_w + dt * tree_sum<W>(pp + (1 + iwa) * kL, NP * kL) * Nt) * rd;
         const double vr = (old_r + dt * tree_sum<W>(pp + (1 + irim) * kL, NP * kL) * Nt) * rd;
-        if (act) sRF[(t - Ioff) * kL + lane] = rime(nn, vw, vr);
+        if (act) sRF[(t - Ioff) * kL + lane] = rime(nn, nlim_t, vw, vr);
       }
     }
     for (int q = wv; q <= nu; q += W) {
