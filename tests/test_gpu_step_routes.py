@@ -271,3 +271,36 @@ def test_one_lane_step_takes_the_layouts_ice_limit(capi, prec):
         rms = np.sqrt(np.mean(y * y, axis=1, keepdims=True))
         bad = ~(np.abs(x - y) <= 1e-9 * np.abs(y) + 1e-12 * rms + 10. * np.abs(y - y2))
         assert not bad.any(), (np.argwhere(bad)[:3], x[bad][:3], y[bad][:3], y2[bad][:3])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("level,grid", [(4, (23, 8, 7)), (5, (23, 8, 7)), (5, (23, 11, 12))])
+def test_small_grids_with_nan_in_inactive_bins(capi, level, grid, prec):
+    """A cell without active hydrometeors steps the same in the one launch of a small
+    grid as in the launch of its cost class, whatever its inactive bins hold: bit
+    for bit at the same lanes per cell, NaN and negative masses among them."""
+    print("case small grid with NaN in inactive bins, level %d grid %s prec %d" % (level, grid, prec), flush=True)
+    desc, f = fields(capi, ("SO4", "DU"), level, grid)
+    g, ncat = f.grid, 4 if level == 5 else 3
+    idx = g.interior_index()
+    n, m = [x.copy() for x in f.n[:ncat]], [x.copy() for x in f.m[:ncat]]
+    for c in range(1, ncat):
+        n[c][:, idx[::2]] = 0.
+        m[c][:, idx[::2]] = 0.
+        m[c][0, idx[::4]] = np.nan
+        m[c][-1, idx[::6]] = np.nan
+        m[c][1, idx[::10]] = -1.e-5
+    lanes = 32 if level == 4 else 64 if g.ncells <= 2048 else 16
+    res = []
+    for shape in (0, lanes):
+        ctx = capi.Context(desc, capi.params(level=level, precision=prec), g.nzp, g.nxp, g.nyp)
+        for k in range(3 if shape else 0):
+            ctx.set_shape(k, shape)
+        a, b = [x.copy() for x in n], [x.copy() for x in m]
+        fd = {k: np.array(getattr(f, k)) for k in ("press", "temp", "rsl", "rsi", "dn", "rv")}
+        ctx.step_host(fd, a, b, flags=capi.STEP_INPLACE)
+        res.append(([x[:, idx] for x in a + b + [fd["rv"][None]]], ctx.cell_flags()))
+        ctx.close()
+    assert np.array_equal(res[0][1], res[1][1])
+    for x, y in zip(res[0][0], res[1][0]):
+        assert np.array_equal(x, y), np.argwhere(x != y)[:3]

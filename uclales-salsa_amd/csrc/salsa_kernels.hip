@@ -355,6 +355,10 @@ k_salsa_step(const DevLayout *__restrict__ Dp, StepArgs a, SmemGeom G) {
       }
     }
     abits = cell_or64<L>(abits);
+    // With kernels of this step a cell without active hydrometeors takes the
+    // aerosol entries alone, as in the other variant: the others' kernels are
+    // zero, but what their bins hold may be NaN.
+    const bool dry = HYD && !a.kmode && !(abits >> D.nb[0]);
     __syncthreads();
 
     // ---- 3. pairs (buildKernelSelf / buildKernel, kernels.f90:94-180) ----
@@ -431,7 +435,7 @@ k_salsa_step(const DevLayout *__restrict__ Dp, StepArgs a, SmemGeom G) {
       const int nu = (fl & TF_ICE) ? nspec : TG.nupd;
       const int nupd = TG.nupd;
       const uint32_t *ent = tent + TG.ent0;
-      const int ne = HYD ? TG.nent : TG.nent_aero;
+      const int ne = HYD && !dry ? TG.nent : TG.nent_aero;
 
       double sink = 0., so = 0., sx = 0., src[NS];
 #pragma unroll
