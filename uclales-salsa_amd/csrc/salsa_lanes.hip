@@ -51,8 +51,7 @@ namespace {
 // The sweep program: per target and wavefront 32 words, one per lane of a
 // register, taken from there by lane number (the loop over the targets then
 // has no scalar loads, whose waits would be shared with those on LDS).
-__host__ __device__ constexpr int prog_entries(int W) { return W == 16 ? 4 : 8; }   // words 0..: entries:
-                                              // pair << 15 | bin << 9 | roles
+constexpr int kEnt = 8;                       // words 0..: entries: pair << 15 | bin << 9 | roles
 constexpr int kProgT = 8, kProgK = 9, kProgN = 10, kProgS = 12, kProgQ = 13;   // target | flags << 8; pair of its
                                               // self term; nlim (two words); cloud-cloud pair of its self-
                                               // collection, -1 without; parity of the first quad (below)
@@ -346,18 +345,19 @@ __device__ __forceinline__ double equil_bin(double n, double zcore, double c1, d
 // Sums over a cell's collectors are taken in VL partial sums, entry e in
 // partial e % VL, which are then added as a balanced tree; a wavefront holds
 // VL / W neighbouring partials and adds them before the W wavefronts' sums
-// meet.  With VL = 16 or 32 that is the order of the general kernel's 16 or 32
-// lanes per cell, bit for bit.
+// meet.  With VL = 16 or 32 that is the order of the general kernel's sums at 16
+// or 32 lanes per cell: 94 % of the cells of a level-5 step with ice everywhere
+// then have its bits (FP64 with dust 32 %), the others differ by rounding in
+// products that the compiler contracts otherwise.
 template <int W>
 __device__ __forceinline__ double tree_sum(const double *p, int stride) {
-  static_assert(W == 4 || W == 8 || W == 16, "wavefronts per workgroup");
+  static_assert(W == 4 || W == 8, "wavefronts per workgroup");
   double q[W / 4];
 #pragma unroll
   for (int v = 0; v < W / 4; ++v)
     q[v] = (p[(4 * v) * stride] + p[(4 * v + 1) * stride]) + (p[(4 * v + 2) * stride] + p[(4 * v + 3) * stride]);
   if constexpr (W == 4) return q[0];
-  else if constexpr (W == 8) return q[0] + q[1];
-  else return (q[0] + q[1]) + (q[2] + q[3]);
+  else return q[0] + q[1];
 }
 // the same over the V values of each of a cell's VL / V lanes
 template <int VL, int V>
@@ -377,12 +377,10 @@ __host__ __device__ inline int sweep_lds(int nb, int NV, int W, int ncc, int nic
 }
 
 // wavefronts per SIMD that the LDS of a shape leaves room for
-__host__ __device__ constexpr int sweep_waves(bool hyd, int NV, int W) {
-  return !hyd ? 4 : NV == 2 ? (W == 4 ? 3 : 4) : W / 4;
-}
+__host__ __device__ constexpr int sweep_waves(bool hyd, int NV) { return !hyd ? 4 : NV == 2 ? 3 : 2; }
 
 template <class KT, int NV, bool L5, int W, int VL, int NR, bool HYD>
-__global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep(const DevLayout *__restrict__ Dp, StepArgs a,
+__global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV)) k_lanes_sweep(const DevLayout *__restrict__ Dp, StepArgs a,
                                                                         LanesArgs w) {
   extern __shared__ __align__(16) char smem[];
   const DevLayout &D = *Dp;
@@ -390,7 +388,6 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
   constexpr int V = VL / W, NQ = V * NR;      // substeps, W lanes per cell: partial sums and bins per lane
   constexpr int NC = 1 + NV;                  // components of a bin's state: number, volumes
   constexpr int NP = sweep_parts(NV), NF = HYD ? prog_pf(VL) : 1;
-  constexpr int kEnt = prog_entries(W);
   constexpr int nwet = L5 ? NV - 1 : NV, ndry = nwet - 1, iwa = nwet - 1, irim = NV - 1;
   const int lane = threadIdx.x & 63, wv = wave_id();
   const int nb = HYD ? D.nt : D.nb[0], ncc = HYD ? D.ncc : 0;
@@ -733,7 +730,6 @@ __global__ void __launch_bounds__(64 * W, sweep_waves(HYD, NV, W)) k_lanes_sweep
       }
       if constexpr (VL == 32) return ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
       else if constexpr (VL == 16) return (y[0] + y[1]) + (y[2] + y[3]);
-      else if constexpr (VL == 8) return y[0] + y[1];
       else return y[0];
     };
     double w1 = 0.;
@@ -1090,7 +1086,6 @@ inline int lanes_volumes(const DevLayout &L) { return L.level == 5 ? L.nspec : L
 // tree, and the parity of that quad says how the (up to three) quads add up.
 int sweep_program(const DevLayout &L, int kt, bool hyd, uint32_t *prog) {
   const int NV = lanes_volumes(L), W = !hyd ? kWavesA : NV > 2 ? kWaves4 : kWaves2, VL = !hyd ? kPartA : NV == 2 ? kPart2 : L.level == 5 && kt == 8 ? kPart5d : kPart4, A = VL / W;
-  const int kEnt = prog_entries(W);
   const int i0 = hyd ? 0 : L.it_aero0, nt = hyd ? L.ntarget : L.it_aero1 - L.it_aero0;
   const uint32_t zero = hyd ? L.npair : L.npair_aa;
   if (zero > 1023u || nt < 1) return -1;
