@@ -502,9 +502,13 @@ static bool lanes_ready(salsa_ctx *c) {
   // list fills the chip for long.  Measured us, one after the other / side by
   // side: level 4 mixed 15 360 cells 246 / 192, 40 960 269 / 213, 81 920
   // 356 / 339, with drizzle 362 / 260, FP64 433 / 398, 176 715 797 / 767; the
-  // deck of 491 520 cells 1 317 / 1 335; level 5 with ice everywhere (an empty
-  // second list) 10 240 255 / 259.
-  if (ok && c->hostL.level == 4 && c->ncells <= (1 << 18))
+  // deck of 491 520 cells 1 317 / 1 335.  Level 5 with ice in 30 % of the cells
+  // mixed 5 120 301 / 238, 10 240 307 / 243, FP64 324 / 250, 329 / 254 (launches
+  // by cost class 280, 327, 291, 348); with ice everywhere or nowhere, where one
+  // list is empty, the second stream costs 5 or 17 (mixed 5 120 231 / 236 and
+  // 112 / 128): taken where the lists one after the other are slower than by
+  // class, to 12 288 cells (30 720 with ice in 30 %: 336 and by class 616).
+  if (ok && c->ncells <= (c->hostL.level == 5 ? 12288 : 1 << 18))
     ok = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) == hipSuccess &&
          hipEventCreateWithFlags(&c->join, hipEventDisableTiming) == hipSuccess;

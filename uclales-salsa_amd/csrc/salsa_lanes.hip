@@ -1138,12 +1138,16 @@ constexpr int kSlotsHyd = 1 << 17, kSlotsAero = 1 << 19;
 // The fewest cells of a context that steps with one lane per cell.  A
 // workgroup here takes as long for its 64 cells as for one, about 0.1 ms for a
 // sweep, and the chip is filled from 256 workgroups on; 16 to 64 lanes per
-// cell share the work of a few cells.  Measured us, here / the general kernel
-// on all cells in one launch: level 4 (32 lanes) mixed 5 120 cells 239 / 134,
-// 10 240 243 / 202, 15 360 246 / 266, with drizzle 10 240 261 / 215, 15 360
-// 264 / 275, FP64 10 240 252 / 220, 15 360 255 / 292.  Level 5 (16 lanes)
-// mixed 3 840 cells 239 / 200, 5 120 242 / 224, 10 240 254 / 396, FP64 3 840
-// 254 / 212, 5 120 253 / 376: more than one wavefront per SIMD.
+// cell share the work of a few cells.  Measured us, here (both lists side by
+// side) / the general kernel on all cells in one launch: level 4 (32 lanes)
+// mixed 5 120 cells 183 / 133, 7 680 186 / 183, 10 240 189 / 201, 15 360
+// 190 / 266, with drizzle 7 680 202 / 196, 10 240 205 / 226, 15 360 206 / 293, FP64
+// 5 120 180 / 144, 7 680 182 / 198, 15 360 184 / 292: the line would pay from 10 240 on,
+// it lies where it paid with the lists one after the other (246 / 266).  Level 5
+// (16 lanes) with ice in 30 % of the cells mixed 5 120 238 / 210, 10 240
+// 243 / 351, FP64 3 840 320 (one after the other) / 194, 5 120 250 / 319; with ice
+// everywhere mixed 3 840 228 / 188, 5 120 236 / 211, 10 240 249 / 372, FP64
+// 3 840 247 / 200, 5 120 253 / 348: more than one wavefront per SIMD.
 int64_t lanes_least(const DevLayout &L) { return L.level == 5 ? 4096 : 15360; }
 
 // Whether the lane kernels take a context of ncells cells with this layout.
