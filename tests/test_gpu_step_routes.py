@@ -137,10 +137,11 @@ def test_only_steps_take_the_step_work_space(capi):
     ctx.close()
 
 
-@pytest.mark.parametrize("level,grid", [(4, (40, 16, 25)), (5, (40, 11, 11))])
+@pytest.mark.parametrize("level,grid", [(4, (40, 16, 25)), (5, (40, 11, 11)), (4, (30, 8, 8)), (4, (39, 19, 20))])
 def test_first_step_of_a_context_within_a_capture(capi, level, grid):
-    """The first step makes its work space also within a stream capture; replays,
-    with other work between them, give the bits of an eager step."""
+    """The first step makes its work space also within a stream capture, and grids
+    that go by cost class otherwise take one launch there; replays, with other
+    work between them, give the bits of an eager step."""
     import torch
     print("case first step captured, level %d" % level, flush=True)
     desc, f = fields(capi, ("SO4",), level, grid)

@@ -446,19 +446,27 @@ static int launch_class(salsa_ctx *c, int k, const StepArgs &a, hipStream_t s, i
 // Lanes per cell with which a small context runs all its cells in one launch
 // of the variant for hydrometeors; 0 where it goes by cost class.  Classes
 // save work on dry cells, but cost three small kernels, a wait for the counts
-// and launches that follow each other, each as long as its slowest cell: below
-// the size from which one lane per cell pays, the chip has room for every cell
-// at once.  Measured us by class / in one launch: level 4 (32 lanes) mixed
-// 640 cells 198 / 108, 2 560 204 / 119, 10 240 231 / 202, FP64 204 / 113,
-// 208 / 126, 246 / 220; level 5 mixed 640 172 / 152 (64 lanes), 2 560
-// 214 / 193 (64) and 196 (16), 3 840 214 / 256 (64) and 200 (16), FP64 175 /
-// 155, 225 / 204 and 208, 234 / 269 and 212.
+// and launches that follow each other, each as long as its slowest cell: while
+// the chip has room for every cell at once, one launch is faster.  Measured us
+// by class (tuned shapes) / in one launch: level 4 (32 lanes) mixed 2 560 cells
+// 205 / 118, 10 240 239 / 200, 14 080 266 / 253, with drizzle 10 240 249 / 225,
+// 14 080 284 / 276, 14 820 281 / 286, FP64 2 560 208 / 125, 10 240 244 / 220,
+// with drizzle 10 240 264 / 258, 11 520 269 / 274, 14 820 306 / 329; level 5 mixed
+// 640 163 / 142 (64 lanes), 2 560 202 / 184 (16), 3 840 205 / 188, FP64 166 / 147,
+// 214 / 196, 218 / 200 (16 against 64 lanes: 2 560 mixed 196 / 193, 3 840
+// 200 / 256).  Within a stream capture, where no count can be waited for, all
+// sizes take one launch.
 // The kernel store (kmode) keeps its cells in list order and stays by class.
 static int direct_lanes(const salsa_ctx *c, const StepArgs &a) {
   if (c->shape_set || a.kmode || c->ncells >= lanes_least(c->hostL)) return 0;
-  const int lanes = c->hostL.level == 5 ? (c->ncells <= 2048 ? 64 : 16) : 32;
+  const bool l5 = c->hostL.level == 5, fp64 = c->params.precision == SALSA_FP64;
+  if (!l5 && c->ncells > (fp64 ? 11264 : 14336)) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &st) != hipSuccess || st == hipStreamCaptureStatusNone) return 0;
+  }
+  const int lanes = l5 ? (c->ncells <= 2048 ? 64 : 16) : 32;
   SmemGeom G;
-  return make_geom(c->hostL, true, c->params.precision == SALSA_FP64 ? 8 : 4, lanes, a.rates != nullptr, G) ? 0 : lanes;
+  return make_geom(c->hostL, true, fp64 ? 8 : 4, lanes, a.rates != nullptr, G) ? 0 : lanes;
 }
 
 // Gather + classification, then the class counts to the host (they size the
