@@ -313,6 +313,26 @@ extern "C" int salsa_ctx_create(const salsa_bin_desc *desc, const salsa_params *
       set_error("copy of the sweep program failed");
       return fail(SALSA_ERR_HIP);
     }
+    // The cells with and without hydrometeors run side by side where neither
+    // list fills the chip for long.  Measured us, one after the other / side by
+    // side: level 4 mixed 15 360 cells 246 / 192, 40 960 269 / 213, 81 920
+    // 356 / 339, with drizzle 362 / 260, FP64 433 / 398, 176 715 797 / 767; the
+    // deck of 491 520 cells 1 317 / 1 335.  Level 5 with ice in 30 % of the cells
+    // mixed 5 120 301 / 238, 10 240 307 / 243, FP64 324 / 250, 329 / 254 (launches
+    // by cost class 280, 327, 291, 348); with ice everywhere or nowhere, where one
+    // list is empty, the second stream costs 5 or 17 (mixed 5 120 231 / 236 and
+    // 112 / 128): taken where the lists one after the other are slower than by
+    // class, to 12 288 cells (30 720 with ice in 30 %: 336 and by class 616).
+    // The second stream is made right after the first: streams take the few
+    // hardware queues in turn, and on one queue the lists would run one after the
+    // other (176 715 cells FP64 826 instead of 768).
+    if (c->ncells <= (c->hostL.level == 5 ? 12288 : 1 << 18) &&
+        (hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
+         hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) != hipSuccess ||
+         hipEventCreateWithFlags(&c->join, hipEventDisableTiming) != hipSuccess)) {
+      set_error("hipStreamCreate failed");
+      return fail(SALSA_ERR_HIP);
+    }
   }
   if (hipMemcpy(c->devL, &c->hostL, sizeof(DevLayout), hipMemcpyHostToDevice) != hipSuccess) {
     set_error("copy of device tables failed"); return fail(SALSA_ERR_HIP);
@@ -498,32 +518,17 @@ static StepArgs class_args(salsa_ctx *c, const StepArgs &a, int k) {
 // is no memory for it.
 static bool lanes_ready(salsa_ctx *c) {
   if (c->lanes_buf || c->lanes_none) return c->lanes_buf;
-  // Allocations, a stream and events leave a capture as it is.
+  // An allocation leaves a capture as it is.
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
   LanesArgs &w = c->lw;
   std::memset(&w, 0, sizeof(w));
   const int kt = c->params.precision == SALSA_FP64 ? 8 : 4;
   const size_t need = lanes_work(c->hostL, kt, c->ncells, w);
-  bool ok = hipMalloc(&c->lanes_buf, need) == hipSuccess;
-  // The cells with and without hydrometeors run side by side where neither
-  // list fills the chip for long.  Measured us, one after the other / side by
-  // side: level 4 mixed 15 360 cells 246 / 192, 40 960 269 / 213, 81 920
-  // 356 / 339, with drizzle 362 / 260, FP64 433 / 398, 176 715 797 / 767; the
-  // deck of 491 520 cells 1 317 / 1 335.  Level 5 with ice in 30 % of the cells
-  // mixed 5 120 301 / 238, 10 240 307 / 243, FP64 324 / 250, 329 / 254 (launches
-  // by cost class 280, 327, 291, 348); with ice everywhere or nowhere, where one
-  // list is empty, the second stream costs 5 or 17 (mixed 5 120 231 / 236 and
-  // 112 / 128): taken where the lists one after the other are slower than by
-  // class, to 12 288 cells (30 720 with ice in 30 %: 336 and by class 616).
-  if (ok && c->ncells <= (c->hostL.level == 5 ? 12288 : 1 << 18))
-    ok = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) == hipSuccess &&
-         hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) == hipSuccess &&
-         hipEventCreateWithFlags(&c->join, hipEventDisableTiming) == hipSuccess;
+  const bool ok = hipMalloc(&c->lanes_buf, need) == hipSuccess;
   if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
   if (!ok) {
     (void)hipGetLastError();                  // not an error of the step, which the general kernel takes
-    (void)hipFree(c->lanes_buf);
     c->lanes_buf = nullptr;
     c->lanes_none = true;
     return false;
