@@ -345,7 +345,15 @@ int salsa_gradient_device_noalloc(salsa_ctx *ctx, const double *press, const dou
  * store or initialization), and smaller ones in one launch of 16 to 64 lanes
  * per cell; the shapes then count for the other calls, and
  * salsa_set_launch_shape with a new value selects launches by cost class with
- * the shapes for every call of the context. */
+ * the shapes for every call of the context, also after salsa_autotune.
+ * These routes take the same sums in other orders: a cell's result differs
+ * between them by rounding, which dusty cells near 273 K at level 5 can grow to
+ * 1e-7 of an element within two steps.  A domain whose parts take other routes than
+ * the whole, or a run that asks for rate fields in some steps, therefore agrees
+ * to rounding, not in bits; a launch shape set for every context fixes the route.
+ * The first step with one lane per cell allocates its work space (up to 0.4 GB
+ * of the default 26-bin layout in mixed precision, 0.7 GB in FP64); without
+ * memory for it the launches by cost class take the step. */
 /*
  * The LES side of a SALSA step for the SALSA tracers, on device: what cfll
  * runs after run_SALSA (step.f90:330-333) -- tend_constrain2
@@ -423,13 +431,17 @@ int salsa_autotune(salsa_ctx *ctx, const double *press, const double *temp,
  * resets and enables it: each step then records one event before its first and
  * one after its last step-kernel launch.  salsa_ctx_kernel_time waits for the
  * stream and returns the summed milliseconds and the number of steps timed.
+ * (Timed steps with one lane per cell run the cells without and with
+ * hydrometeors one after the other; untimed ones may run them side by side.)
  * (Instrumentation with no counterpart in the reference, which only prints
  * cpu_time per LES step, step.f90:134-141.) */
 int salsa_ctx_timing(salsa_ctx *ctx, int32_t enable);
 int salsa_ctx_kernel_time(salsa_ctx *ctx, double *ms, int64_t *nsteps);
 /* The same events split by launch, summed over the timed steps: ms[0] gather
  * and cost classification, ms[1..3] the step kernel of cost class 0, 1, 2,
- * ms[4] scatter; cells[0..2] the cells each class kernel processed.  Each
+ * ms[4] scatter; cells[0..2] the cells each class kernel processed (all in
+ * cells[2] where one launch takes every cell; with one lane per cell classes 0
+ * and 1 share a launch, whose time is divided by their cells).  Each
  * figure spans only its own launches (the class-count read-back between the
  * classification and the class kernels is outside every span). */
 int salsa_ctx_phase_time(salsa_ctx *ctx, double ms[5], int64_t cells[3], int64_t *nsteps);

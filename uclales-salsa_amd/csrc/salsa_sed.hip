@@ -364,7 +364,7 @@ __host__ __device__ inline size_t sed_prc_lds_bytes(int Z, int nb, int ns, int M
 // scans the sources above it once for all quantities.  With a barrier and a
 // scan per bin and moved quantity (35 and 21 of them) the ice launch took 929 us
 // at 128 x 128 x 100 cells and the precipitation launch 127 us at 64 x 64 x 120;
-// now 707 and 108 us, with the fall speeds' bits as they were.  (Reciprocals
+// now 694 and 106 us, with the fall speeds' bits as they were.  (Reciprocals
 // without sd_quot's correction: 617 and 98 us, but fall speeds further from the
 // exact value, 5.3 against 4.6 units of 2^-53 rms.  Four wavefronts per SIMD,
 // with 14 to 34 spills, 698 and 124 us before the ice speed took its
